@@ -350,6 +350,7 @@ Engine::Engine(const HostModel& model, const EngineOptions& options) : params_(m
     const uint32_t G = p.n_head / p.n_head_kv;
     const uint32_t attn_rows = static_cast<uint32_t>(gpu::attention_max_rows(static_cast<int32_t>(p.head_dim)));
     prefill_chunk_ = std::max<uint32_t>(1, std::min<uint32_t>(gpu::kMaxRows, attn_rows / G));
+    if (p.head_dim == 64 || p.head_dim == 128) prefill_chunk_ = gpu::kPrefillRows;
 
     if (p.head_dim % 4 != 0) fail(Status::InvalidArgument, "head dimension must be a multiple of 4");
     if (p.n_ff % gpu::kGluGroup != 0) fail(Status::InvalidArgument, "feed-forward length must be a multiple of 8");
@@ -432,15 +433,15 @@ Engine::Engine(const HostModel& model, const EngineOptions& options) : params_(m
     }
 
     const int32_t H = static_cast<int32_t>(p.n_embd), F = static_cast<int32_t>(p.n_ff);
-    const size_t R = gpu::kMaxRows;
+    const size_t R = std::max<size_t>(gpu::kMaxRows, prefill_chunk_), S = gpu::kMaxRows;
     h_ = static_cast<float*>(device_alloc(R * H * sizeof(float)));
     q_ = static_cast<float*>(device_alloc(R * Hq * sizeof(float)));
     attn_ = static_cast<float*>(device_alloc(R * Hq * sizeof(float)));
     ffn_ = static_cast<float*>(device_alloc(R * F * sizeof(float)));
-    if (last_stage()) logits_ = static_cast<float*>(device_alloc(R * static_cast<size_t>(p.n_vocab) * sizeof(float)));
-    best_ = static_cast<unsigned long long*>(device_alloc(R * sizeof(unsigned long long)));
+    if (last_stage()) logits_ = static_cast<float*>(device_alloc(S * static_cast<size_t>(p.n_vocab) * sizeof(float)));
+    best_ = static_cast<unsigned long long*>(device_alloc(S * sizeof(unsigned long long)));
     // argmax slots start cleared; k_embed and k_finish clear them for every step
-    hip_check(hipMemset(best_, 0, R * sizeof(unsigned long long)), "clear argmax slots");
+    hip_check(hipMemset(best_, 0, S * sizeof(unsigned long long)), "clear argmax slots");
     // int8 rows with room for the scales of 32-value blocks (the block size is the consumer's)
     auto act8 = [&](int32_t K, int32_t blk) {
         gpu::Act8 a;
@@ -625,6 +626,8 @@ void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_ou
     };
     // attention split slots this step shape can fill (a prefill chunk: few long splits)
     const int32_t slots = gpu::attention_slots(splits_, attn_capacity_, n_rows, n_seq);
+    const bool whole_keys = gpu::attention_prefill_supported(n_rows, n_seq, static_cast<int32_t>(p.n_head),
+                                                             static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim));
     // l: the resident layer (its slot in the sessions' caches)
     for (uint32_t l = 0; l < layers_.size(); ++l) {
         const Layer& L = layers_[l];
@@ -641,15 +644,25 @@ void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_ou
         qkv.qkv.n_head_kv = static_cast<int32_t>(p.n_head_kv);
         qkv.qkv.head_dim = static_cast<int32_t>(p.head_dim);
         matmul(qkv, "qkv");
-        timed("k_attention", attn_kv_bytes_ + n * Hq * 4.0, [&] {
-            gpu::launch_attention(q_, step_dev_, max_len, n_seq, static_cast<int32_t>(l), static_cast<int32_t>(p.n_head),
-                                  static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim), splits_, partial_, s,
-                                  slots);
-        });
-        timed("k_attention_merge", n * Hq * 4.0 * (slots + 1.0) + (xq_attn_.q ? n * Hq * 1.1 : 0.0), [&] {
-            gpu::launch_attention_merge(partial_, step_dev_, n_rows, static_cast<int32_t>(p.n_head),
-                                        static_cast<int32_t>(p.head_dim), splits_, attn_, xq_attn_, s, slots);
-        });
+        if (whole_keys) {
+            timed("k_attention_prefill", attn_kv_bytes_ + n * Hq * 8.0, [&] {
+                gpu::launch_attention_prefill(q_, step_dev_, n_rows, static_cast<int32_t>(l), static_cast<int32_t>(p.n_head),
+                                              static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim), attn_, s);
+            });
+            if (xq_attn_.q) {
+                timed("k_quantize", n * Hq * 5.1, [&] { gpu::launch_quantize(attn_, Hq, n_rows, xq_attn_, s); });
+            }
+        } else {
+            timed("k_attention", attn_kv_bytes_ + n * Hq * 4.0, [&] {
+                gpu::launch_attention(q_, step_dev_, max_len, n_seq, static_cast<int32_t>(l), static_cast<int32_t>(p.n_head),
+                                      static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim), splits_, partial_, s,
+                                      slots);
+            });
+            timed("k_attention_merge", n * Hq * 4.0 * (slots + 1.0) + (xq_attn_.q ? n * Hq * 1.1 : 0.0), [&] {
+                gpu::launch_attention_merge(partial_, step_dev_, n_rows, static_cast<int32_t>(p.n_head),
+                                            static_cast<int32_t>(p.head_dim), splits_, attn_, xq_attn_, s, slots);
+            });
+        }
         gpu::GemvArgs o;
         o.mat = L.o->mat;
         o.mode = gpu::kAdd;
@@ -779,7 +792,9 @@ std::vector<KernelStat> Engine::profile(const std::vector<SeqStep>& steps, uint3
         options_.use_graphs = false;
         std::vector<int32_t> ids(gpu::kMaxRows);
         for (uint32_t it = 0; it < iterations; ++it) {
-            forward(steps, ids.data(), nullptr, nullptr);
+            // a single sequence's step may be a whole prefill chunk
+            forward(steps, ids.data(), nullptr, nullptr, nullptr, nullptr,
+                    steps.size() == 1 ? std::max<uint32_t>(gpu::kMaxRows, prefill_chunk_) : gpu::kMaxRows);
             for (const SeqStep& st : steps) st.session->position_ -= st.n;
         }
         options_.use_graphs = graphs;
@@ -849,7 +864,7 @@ std::vector<int32_t> Engine::end_tokens() const {
 }
 
 void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits,
-                     float* act_out, PrefillMetrics* metrics) {
+                     float* act_out, PrefillMetrics* metrics, uint32_t row_limit) {
     using clock = std::chrono::steady_clock;
     const auto ms_since = [](clock::time_point t) { return std::chrono::duration<double, std::milli>(clock::now() - t).count(); };
     std::lock_guard lock(mutex_);
@@ -880,10 +895,11 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
         if (static_cast<uint64_t>(s->position_) + st.n > s->capacity_) {
             fail(Status::InvalidArgument, "native Qwen2 step is outside session capacity");
         }
-        if (st.n * G > static_cast<uint32_t>(gpu::attention_max_rows(static_cast<int32_t>(p.head_dim)))) {
+        if (row_limit <= gpu::kMaxRows &&
+            st.n * G > static_cast<uint32_t>(gpu::attention_max_rows(static_cast<int32_t>(p.head_dim)))) {
             fail(Status::InvalidArgument, "too many rows for one sequence step");
         }
-        if (rows + static_cast<int32_t>(st.n) > gpu::kMaxRows) fail(Status::InvalidArgument, "too many token rows in one step");
+        if (static_cast<uint64_t>(rows) + st.n > row_limit) fail(Status::InvalidArgument, "too many token rows in one step");
         sd.seqs[si].k = s->k_;
         sd.seqs[si].v = s->v_;
         sd.seqs[si].capacity = static_cast<int32_t>(s->stride_);
@@ -895,9 +911,10 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
             if (st.tokens && (tok < 0 || static_cast<uint32_t>(tok) >= p.n_vocab)) {
                 fail(Status::InvalidArgument, "native token ID is outside model vocabulary");
             }
-            sd.token[rows + i] = tok;
-            sd.pos[rows + i] = static_cast<int32_t>(s->position_ + i);
-            sd.seq[rows + i] = static_cast<int32_t>(si);
+            sd.rows[rows + i] = {tok, static_cast<int32_t>(s->position_ + i), static_cast<int32_t>(si)};
+        }
+        if (static_cast<uint64_t>(outs) + (st.logits == 2 ? st.n : st.logits) > gpu::kMaxRows) {
+            fail(Status::InvalidArgument, "too many logits rows in one step");
         }
         if (st.logits == 1) {
             sd.out_row[outs] = rows + static_cast<int32_t>(st.n) - 1;
@@ -923,9 +940,10 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
     sd.n_end = static_cast<int32_t>(end_tokens_.size());
     std::copy(end_tokens_.begin(), end_tokens_.end(), sd.end_token);
     const bool store = logits != nullptr && outs > 0;
-    hip_check(hipMemcpyAsync(step_dev_, step_host_, sizeof(gpu::StepDev), hipMemcpyHostToDevice, stream_), "upload step");
+    const size_t step_bytes = offsetof(gpu::StepDev, rows) + static_cast<size_t>(rows) * sizeof(gpu::RowDev);
+    hip_check(hipMemcpyAsync(step_dev_, step_host_, step_bytes, hipMemcpyHostToDevice, stream_), "upload step");
     // input rows of a later stage: the previous stage's residual stream
-    uint64_t input_bytes = sizeof(gpu::StepDev);
+    uint64_t input_bytes = step_bytes;
     for (size_t si = 0; si < steps.size(); ++si) {
         if (steps[si].activations == nullptr) continue;
         const size_t bytes = static_cast<size_t>(steps[si].n) * p.n_embd * sizeof(float);
@@ -940,7 +958,8 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
         metrics->attention_matrix_cores = p.head_dim == 64 || p.head_dim == 128;
         ++metrics->steps;
     }
-    if (options_.use_graphs) {
+    // a long chunk's kernels outlast their launches: no graph is captured for its row count
+    if (options_.use_graphs && rows <= gpu::kMaxRows) {
         const uint64_t key = (static_cast<uint64_t>(rows) << 40) | (static_cast<uint64_t>(max_len) << 32) |
                              (static_cast<uint64_t>(steps.size()) << 16) | (static_cast<uint64_t>(outs) << 1) |
                              (store ? 1u : 0u);
@@ -1033,6 +1052,12 @@ BufferMetrics Engine::buffer_metrics(uint32_t capacity, uint32_t prompt_tokens, 
     return m;
 }
 
+// Rows per chunk of an n-row prefill: as many chunks as needed, about equally long (in whole 128-token groups).
+uint32_t Engine::balanced_chunk(uint32_t n) const {
+    const uint32_t chunks = std::max<uint32_t>(1, (n + prefill_chunk_ - 1) / prefill_chunk_);
+    return std::min(prefill_chunk_, ((n + chunks - 1) / chunks + 127) / 128 * 128);
+}
+
 int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* logits) {
     require_full_model();
     if (s.position_ != 0 || n == 0 || n > s.capacity_) {
@@ -1041,15 +1066,16 @@ int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* lo
     int32_t token = -1;
     PrefillMetrics m;
     m.allocation_ms = s.prefill_metrics_.allocation_ms;
+    const uint32_t chunk = balanced_chunk(n);
     for (uint32_t done = 0; done < n;) {
-        const uint32_t len = std::min(prefill_chunk_, n - done);
+        const uint32_t len = std::min(chunk, n - done);
         const bool last = done + len == n;
         SeqStep st;
         st.session = &s;
         st.tokens = tokens + done;
         st.n = len;
         st.logits = last ? 1 : 0;
-        forward({st}, last ? &token : nullptr, nullptr, last ? logits : nullptr, nullptr, &m);
+        forward({st}, last ? &token : nullptr, nullptr, last ? logits : nullptr, nullptr, &m, prefill_chunk_);
         done += len;
     }
     s.prefill_position_ = n;
@@ -1076,8 +1102,9 @@ int32_t Engine::stage_prefill(Session& s, const int32_t* tokens, const float* ac
     int32_t token = -1;
     PrefillMetrics m;
     m.allocation_ms = s.prefill_metrics_.allocation_ms;
+    const uint32_t chunk = balanced_chunk(n);
     for (uint32_t done = 0; done < n;) {
-        const uint32_t len = std::min(prefill_chunk_, n - done);
+        const uint32_t len = std::min(chunk, n - done);
         const bool last = done + len == n;
         SeqStep st;
         st.session = &s;
@@ -1086,7 +1113,7 @@ int32_t Engine::stage_prefill(Session& s, const int32_t* tokens, const float* ac
         st.n = len;
         st.logits = last && last_stage() ? 1 : 0;
         forward({st}, st.logits ? &token : nullptr, nullptr, st.logits ? logits : nullptr,
-                act_out ? act_out + done * H : nullptr, &m);
+                act_out ? act_out + done * H : nullptr, &m, prefill_chunk_);
         done += len;
     }
     s.prefill_position_ = n;

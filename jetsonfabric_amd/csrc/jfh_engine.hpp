@@ -143,9 +143,11 @@ public:
     // sequence; logits (optional) n_logits_rows x vocab floats. A stage
     // that is not the last one computes no logits: act_out receives the
     // residual-stream rows after its last layer, f32 [rows][n_embd].
-    // metrics (optional) accumulates the step's host and device times.
+    // metrics (optional) accumulates the step's host and device times. A step has
+    // at most row_limit rows (a prefill chunk of one sequence up to
+    // max_prefill_chunk).
     void forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits,
-                 float* act_out = nullptr, PrefillMetrics* metrics = nullptr);
+                 float* act_out = nullptr, PrefillMetrics* metrics = nullptr, uint32_t row_limit = gpu::kMaxRows);
 
     // Prefill of arbitrary length: runs the prompt in chunks and returns the
     // greedy token of the last row (and its logits if requested).
@@ -229,6 +231,7 @@ private:
     const TensorRef& find_ref(const std::string& name) const;
     const float* upload_f32(const TensorView& t);
     void ensure_capacity(uint32_t capacity);
+    uint32_t balanced_chunk(uint32_t n) const;
     void record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits);
     template <typename F>
     void timed(const std::string& label, double bytes, F&& fn);

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void k_embed(DMat table, const StepDev* step, 
     }
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (r < step->n_rows && c < H) {
-        h[static_cast<size_t>(r) * H + c] = dequant_elem(table, static_cast<uint32_t>(step->token[r]), c);
+        h[static_cast<size_t>(r) * H + c] = dequant_elem(table, static_cast<uint32_t>(step->rows[r].token), c);
     }
 }
 
@@ -1172,8 +1172,9 @@ struct QkvRow {
 
 __device__ __forceinline__ QkvRow qkv_row(const QkvOut& o, int t) {
     const StepDev* st = o.step;
-    const SeqDev& sd = st->seqs[st->seq[o.row0 + t]];
-    return QkvRow{st->pos[o.row0 + t], sd.capacity, sd.k, sd.v};
+    const RowDev row = st->rows[o.row0 + t];
+    const SeqDev& sd = st->seqs[row.seq];
+    return QkvRow{row.pos, sd.capacity, sd.k, sd.v};
 }
 
 #pragma clang fp contract(off)
@@ -2059,129 +2060,8 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_wide(GemvArgs a, int32_t n_rg
     }
 }
 
-// The wide matmul of the K-quant formats (Q4_K, Q6_K, Q2_K, whose tiles keep
-// one accumulator per (row, token): the integer totals of a tile take one
-// float step) over R consecutive 16-row groups per work-group: a wave loads
-// its K tile's activations once for the group's token tiles and runs them
-// against the R row groups' weight tiles (the next row group's tile in flight
-// while the current one is multiplied), so the activation rows are read from
-// L2 once per R row groups instead of once per row group. Per (row, token) the
-// sum is the one-row-group kernel's: each wave's tiles in K order, the waves
-// in order (the lane groups' other accumulators are exact zeros, and adding
-// them to a sum that starts at +0 changes no bit), so rows stay bit-identical
-// to decode rows.
-template <uint32_t TYPE, int R, int TP, bool A32>
-__global__ __launch_bounds__(kMmThreads) void k_mm_wide_rg(GemvArgs a, int32_t n_rg, int32_t tpw) {
-    using T = WideTile<TYPE>;
-    constexpr int W = kMmWaves;
-    constexpr uint32_t TB = tile_bytes(TYPE);
-    __shared__ float red[W][TP][16][16];  // [wave][token tile][token][row] of one row group
-    __shared__ float vals[16 * TP][16 * R];
-    __shared__ u32x4 stage_s[W][TP][16][2];
-    __shared__ float stage_d[W][TP][A32 ? 16 * 8 : 16];  // scales [token] (A32: [token][8])
-    const int n_tok = a.n_tok, n_tt = (n_tok + 15) / 16, n_grp = (n_tt + tpw - 1) / tpw;
-    // work-group k runs on XCD k % 8: the token groups of one row-group set share an XCD (and its L2)
-    const int q = static_cast<int>(blockIdx.x) >> 3;
-    const int grp = q % n_grp, set = (q / n_grp) * 8 + static_cast<int>(blockIdx.x & 7u);
-    const int rg0 = set * R;
-    if (rg0 >= n_rg) return;
-    const int nrg = min(R, n_rg - rg0);
-    const int K = static_cast<int>(a.mat.cols), nb = K / 256;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-    const int i = lane & 15, G = lane >> 4;
-    const int tt0 = grp * tpw, ntl = min(TP, min(n_tt, tt0 + tpw) - tt0);
-    const int t0 = 16 * tt0, nt = min(16 * (tt0 + ntl), n_tok) - t0;
-    const GemvArgs out = token_slice(a, t0, nt);
-    const Act8 xq = a.xq;
-    auto load_act = [&](int tt, int b) { return wide_load_act<T::kSums, A32>(xq, tt, b, n_tok, K, lane); };
-    const uint8_t* base = a.mat.data + static_cast<size_t>(rg0) * nb * TB;
-    float acc[R][TP][4][4];
-#pragma unroll
-    for (int rr = 0; rr < R; ++rr) {
-#pragma unroll
-        for (int tl = 0; tl < TP; ++tl) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[rr][tl][g][j] = 0.0F;
-            }
-        }
-    }
-    for (int b = wave; b < nb; b += W) {
-        // the first row group's tile, then the token tiles' activations (clamped: issued unconditionally)
-        typename T::Wt w = T::load_w(base + static_cast<size_t>(b) * TB, i, G);
-        long av[TP][8];
-        float xd[TP][4];
-        typename T::Xt x[TP];
-#pragma unroll
-        for (int tl = 0; tl < TP; ++tl) {
-            const WideAct r = load_act(tt0 + min(tl, ntl - 1), b);
-            wide_stage<T::kSums, A32>(r, lane, &stage_s[wave][tl][0][0], stage_d[wave][tl]);
-            wide_a_operands(r.xa, av[tl]);
-        }
-        __builtin_amdgcn_wave_barrier();
-        if constexpr (!A32) {
-#pragma unroll
-            for (int tl = 0; tl < TP; ++tl) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) xd[tl][j] = stage_d[wave][tl][4 * G + j];
-                x[tl] = T::load_x(reinterpret_cast<const uint32_t*>(&stage_s[wave][tl][i][0]), G);
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-#pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-            // the next row group's tile (clamped to the group's last) is requested before this one runs
-            const typename T::Wt wn =
-                T::load_w(base + (static_cast<size_t>(min(rr + 1, nrg - 1)) * nb + b) * TB, i, G);
-            if (rr < nrg) {
-#pragma unroll
-                for (int tl = 0; tl < TP; ++tl) {
-                    if (tl < ntl) {
-                        if constexpr (A32) {
-                            T::accumulate32(w, av[tl], reinterpret_cast<const uint32_t*>(&stage_s[wave][tl][0][0]),
-                                            stage_d[wave][tl], G, acc[rr][tl]);
-                        } else {
-                            T::accumulate(w, av[tl], x[tl], xd[tl], G, acc[rr][tl]);
-                        }
-                    }
-                }
-            }
-            w = wn;
-        }
-        // the staged sums and scales are read until the last row group has run
-        if constexpr (A32) __builtin_amdgcn_wave_barrier();
-    }
-    // per row group and token tile: the sum over waves in wave order
-#pragma unroll
-    for (int rr = 0; rr < R; ++rr) {
-        if (rr < nrg) {
-            __syncthreads();
-#pragma unroll
-            for (int tl = 0; tl < TP; ++tl) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) red[wave][tl][4 * G + j][i] = acc[rr][tl][0][j];
-            }
-            __syncthreads();
-            for (int e = threadIdx.x; e < ntl * 256; e += kMmThreads) {
-                const int tl = e >> 8, tk = (e >> 4) & 15, r = e & 15;
-                float v = 0.0F;
-#pragma unroll
-                for (int w2 = 0; w2 < W; ++w2) v += red[w2][tl][tk][r];
-                vals[16 * tl + tk][16 * rr + r] = v;
-            }
-        }
-    }
-    __syncthreads();
-    const int row0 = rg0 * 16;
-    const int nrows = min(16 * nrg, static_cast<int>(a.mat.rows) - row0);
-    gemv_epilogue<kMmThreads, kNoLogits>(out, row0, nrows, [&](int j, int t) { return vals[t][j]; },
-                                         &red[0][0][0][0]);
-}
-
-// The wide Q4_K matmul for steps with many row groups (the gate / up matrix
-// of a prefill chunk): the sub-block scales are folded into the weight
+// The wide Q4_K matmul for steps of 9..32 rows against many row groups (the
+// gate / up matrix of a verify step): the sub-block scales are folded into the weight
 // operand, each wave owns one 16-row group over the whole of K, and the
 // work-group's waves share every activation tile through LDS.
 //
@@ -2209,13 +2089,8 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_wide_rg(GemvArgs a, int32_t n
 //
 // Staging: the work-group's token rows of the next K tile (codes, 16-value
 // sums, scales) are written to the other of two LDS buffers; one barrier per
-// tile. With four token tiles per work-group (long steps) the next tile's
-// staging loads are issued after the current tile's work and a wave loads
-// its weight tile when the tile starts: no register is held across a tile
-// for the next one, so four work-groups fit on a CU (128 VGPRs, 39 KB of LDS
-// each), whose waves hide each other's load latency. With one or two token
-// tiles (9..32-row steps) a tile's work is short, and both loads are issued
-// one tile ahead.
+// tile. A tile's work is short, so both its loads and the next weight tile's
+// are issued one tile ahead.
 constexpr int kStageRow = 272;  // bytes per staged token row: 256 codes + 16 bytes of padding (banks)
 
 template <int NW, int TP>
@@ -2317,24 +2192,15 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
 #pragma unroll
         for (int j = 0; j < 4; ++j) total[tl][j] = chain[tl][j] = 0.0F;
     }
-    // one or two token tiles: the next tile's loads are issued before this tile's work (a short
-    // tile hides little latency); four: after it, so that no register is held across a tile
-    constexpr bool AHEAD = TP < 4;
     stage_store(stage_load(0), 0);
-    Raw ahead{};
-    if constexpr (AHEAD) ahead = load_raw(0);
+    Raw cur = load_raw(0);
     __syncthreads();
     int b = 0;
     for (int s = 0; s < nb; ++s) {
         const int buf = s & 1;
         const int bn = s + 1 < nb ? next_tile(b) : b;  // clamped: issued unconditionally
-        Stage st{};
-        Raw nxt{};
-        if constexpr (AHEAD) {
-            st = stage_load(bn);
-            nxt = load_raw(bn);
-        }
-        const Raw cur = AHEAD ? ahead : load_raw(b);
+        const Stage st = stage_load(bn);
+        const Raw nxt = load_raw(bn);
         if (active) {
             // lane group G's 24-bit field of row i: sc 2G | sc 2G+1 | m 2G | m 2G+1
             const uint32_t f = __builtin_amdgcn_alignbyte(cur.fw.y, cur.fw.x, (3 * G) & 3);
@@ -2402,14 +2268,8 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
                 }
             }
         }
-        // the next tile's staging loads after this tile's work (their registers are not held across it)
-        if constexpr (AHEAD) {
-            if (s + 1 < nb) stage_store(st, buf ^ 1);
-            ahead = nxt;
-        } else {
-            __builtin_amdgcn_sched_barrier(0);
-            if (s + 1 < nb) stage_store(stage_load(bn), buf ^ 1);
-        }
+        if (s + 1 < nb) stage_store(st, buf ^ 1);
+        cur = nxt;
         b = bn;
         __syncthreads();
     }
@@ -2427,20 +2287,475 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
     gemv_epilogue<NTHR, kNoLogits>(out, row0, nrows, [&](int j, int tk) { return vals[tk * VSTRIDE + j]; }, nullptr);
 }
 
-// The wide Q4_K matmul for steps with fewer row groups (the down, output
-// and qkv matrices of a prefill chunk): the decode matmul's eight waves (wave
-// w takes the K tiles w, w + 8, ...), R consecutive row groups and one
-// 16-token tile per work-group, and the folded-scale tile arithmetic of
-// k_mm_wide_q4k. A wave loads its K tile's activations (lane (i, G): token
-// i's bytes 64 G .. 64 G + 63, its code sums and scale) once and runs them
-// against the R row groups' folded weight operands, the next weight tile in
-// flight while one runs; the waves' partials are summed in wave order through
-// LDS, so every row equals the decode row bit for bit.
-template <int R>
-__global__ __launch_bounds__(kMmThreads) void k_mm_wide_q4r(GemvArgs a, int32_t n_rg) {
+// ------------------------------------------------------------------ long-step matmul
+// The matmul of long steps (prefill chunks). Work-group = kGemmWaves waves x
+// RG consecutive 16-row groups x TP consecutive 16-token tiles: each wave owns
+// its RG row groups over the whole of K, and the waves share every K tile's
+// activations through LDS (double-buffered, one barrier per K tile).
+//
+// Per K tile a wave turns its row groups' codes into int8 matrix operands
+// once, with the sub-block scales folded in, and runs them against all TP
+// token tiles, so that per (16 rows, 16 tokens) only the v_mfma_i32_16x16x64_i8
+// chains and one float step remain; each token operand read from LDS feeds the
+// RG row groups. Folds (all exact, the operands fit an int8):
+//   Q4_K  sc = 8 sh + sl: two chains, total = L + 8 H
+//   Q6_K  p = sc (q - 32), |p| <= 4096, p = 64 h + l: two chains, total = L + 64 H
+//   Q2_K  sc q <= 45: one chain
+// The min sums sum_j m_j S_j (Q4_K, Q2_K) take one v_mfma_f32_16x16x16_f16 over
+// the sixteen 16-value code sums: |S| <= 2032 and m <= 63 are exact in f16 and
+// the totals stay below 2^24. (Two v_mfma_f32_16x16x4f32 would hold the matrix
+// cores four times as long.) Q8_0 keeps its float term per 32-value block.
+//
+// Order: a wave walks the K tiles as the decode waves' chains do (0, 8, 16,
+// ..., then 1, 9, ...), keeping the running partial of the current chain and
+// adding it to the total when the chain ends, so every row equals the decode
+// row bit for bit with no cross-wave reduction.
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kGemmWaves = 4;
+
+__device__ __forceinline__ u16x2 dup16(uint32_t v) {
+    const uint16_t h = static_cast<uint16_t>(v);
+    return u16x2{h, h};
+}
+
+__device__ __forceinline__ uint32_t pk_mul(uint32_t c, u16x2 s) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, c) * s);
+}
+
+template <uint32_t TYPE>
+struct GemmTile;
+
+template <>
+struct GemmTile<11> {
+    static constexpr int kChains = 2, kShift = 3;
+    static constexpr bool kMins = true;
+    struct Raw {
+        uint32_t dd[4];
+        uint2 fw;
+        u32x4 w[2];
+    };
+    struct Scale {
+        float d[4], neg_dmin[4];
+        f16x4 mins;
+    };
+    static __device__ __forceinline__ Raw load(const uint8_t* t, int lane) {
+        const int i = lane & 15, G = lane >> 4;
+        Raw r;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r.dd[j] = *reinterpret_cast<const uint32_t*>(t + 16 * (4 * G + j));
+        r.fw = *reinterpret_cast<const uint2*>(t + 16 * i + 4 + 4 * ((3 * G) >> 2));
+        r.w[0] = *reinterpret_cast<const u32x4*>(t + 256 + 16 * lane);
+        r.w[1] = *reinterpret_cast<const u32x4*>(t + 1280 + 16 * lane);
+        return r;
+    }
+    static __device__ __forceinline__ void fold(const Raw& r, int lane, u32x4 (&B)[2][4], Scale& s) {
+        constexpr uint32_t M4 = 0x0F0F0F0Fu;
+        const int G = lane >> 4;
+        // lane group G's 24-bit field of row i: sc 2G | sc 2G+1 | m 2G | m 2G+1
+        const uint32_t f = __builtin_amdgcn_alignbyte(r.fw.y, r.fw.x, (3 * G) & 3);
+        const _Float16 ma = static_cast<_Float16>(static_cast<uint16_t>((f >> 12) & 63u));
+        const _Float16 mb = static_cast<_Float16>(static_cast<uint16_t>((f >> 18) & 63u));
+        s.mins = f16x4{ma, ma, mb, mb};
+        const u16x2 sl[2] = {dup16(f & 7u), dup16((f >> 6) & 7u)};
+        const u16x2 sh[2] = {dup16((f >> 3) & 7u), dup16((f >> 9) & 7u)};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t w = r.w[c & 1][k], q = (c < 2 ? w : w >> 4) & M4;
+                B[0][c][k] = pk_mul(q, sl[c >> 1]);
+                B[1][c][k] = pk_mul(q, sh[c >> 1]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s.d[j] = h2f(r.dd[j]);
+            s.neg_dmin[j] = h2f((r.dd[j] >> 16) ^ 0x8000u);
+        }
+    }
+    // q4k_term_f with the sign moved into dmin (the same products)
+    static __device__ __forceinline__ float step(float acc, float xd, const Scale& s, int j, int isum, float msum) {
+        return __builtin_fmaf(xd, __builtin_fmaf(s.d[j], static_cast<float>(isum), s.neg_dmin[j] * msum), acc);
+    }
+};
+
+template <>
+struct GemmTile<9> {
+    static constexpr int kChains = 1, kShift = 0;
+    static constexpr bool kMins = true;
+    struct Raw {
+        u32x4 dd;
+        uint32_t sc;
+        u32x4 w;
+    };
+    struct Scale {
+        float d[4], neg_dmin[4];
+        f16x4 mins;
+    };
+    static __device__ __forceinline__ Raw load(const uint8_t* t, int lane) {
+        const int i = lane & 15, G = lane >> 4;
+        Raw r;
+        r.dd = *reinterpret_cast<const u32x4*>(t + 16 * G);
+        r.sc = *reinterpret_cast<const uint32_t*>(t + 64 + 16 * i + 4 * G);
+        r.w = *reinterpret_cast<const u32x4*>(t + 320 + 16 * lane);
+        return r;
+    }
+    static __device__ __forceinline__ void fold(const Raw& r, int, u32x4 (&B)[1][4], Scale& s) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            s.mins[c] = static_cast<_Float16>(static_cast<uint16_t>((r.sc >> (8 * c + 4)) & 0xFu));
+            const u16x2 sc = dup16((r.sc >> (8 * c)) & 0xFu);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) B[0][c][k] = pk_mul((r.w[c] >> (2 * k)) & 0x03030303u, sc);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s.d[j] = h2f(r.dd[j]);
+            s.neg_dmin[j] = h2f((r.dd[j] >> 16) ^ 0x8000u);
+        }
+    }
+    // q4k_term_f with the sign moved into dmin (the same products)
+    static __device__ __forceinline__ float step(float acc, float xd, const Scale& s, int j, int isum, float msum) {
+        return __builtin_fmaf(xd, __builtin_fmaf(s.d[j], static_cast<float>(isum), s.neg_dmin[j] * msum), acc);
+    }
+};
+
+template <>
+struct GemmTile<13> {
+    static constexpr int kChains = 2, kShift = 6;
+    static constexpr bool kMins = false;
+    struct Raw {
+        u32x2 d;
+        uint32_t sc;
+        u32x4 w[3];
+    };
+    struct Scale {
+        float d[4];
+        f16x4 mins;
+    };
+    static __device__ __forceinline__ Raw load(const uint8_t* t, int lane) {
+        const int i = lane & 15, G = lane >> 4;
+        Raw r;
+        r.d = *reinterpret_cast<const u32x2*>(t + 8 * G);
+        r.sc = *reinterpret_cast<const uint32_t*>(t + 32 + 16 * i + 4 * G);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r.w[c] = *reinterpret_cast<const u32x4*>(t + 288 + 1024 * c + 16 * lane);
+        return r;
+    }
+    static __device__ __forceinline__ void fold(const Raw& r, int, u32x4 (&B)[2][4], Scale& s) {
+        constexpr uint32_t M4 = 0x0F0F0F0Fu, M30 = 0x30303030u, MW = 0x00FF00FFu;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int sc = sext8(r.sc >> (8 * c));
+            const u16x2 sv = dup16(static_cast<uint32_t>(sc)), off = dup16(static_cast<uint32_t>(-32 * sc));
+            const uint32_t h = r.w[2][c];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t lw = r.w[c >> 1][2 * (c & 1) + (k >> 1)];
+                const uint32_t hi = k < 2 ? h << (4 - 2 * k) : h >> (2 * k - 4);
+                const uint32_t q = ((k & 1 ? lw >> 4 : lw) & M4) | (hi & M30);
+                // sc (q - 32) of the even and the odd bytes' codes, then the low six bits and the rest of each
+                const u16x2 pe = __builtin_bit_cast(u16x2, q & MW) * sv + off;
+                const u16x2 po = __builtin_bit_cast(u16x2, (q >> 8) & MW) * sv + off;
+                typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+                const i16x2 he = __builtin_bit_cast(i16x2, pe) >> 6, ho = __builtin_bit_cast(i16x2, po) >> 6;
+                // bytes (even 0, odd 0, even 1, odd 1)
+                B[0][c][k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, po), __builtin_bit_cast(uint32_t, pe),
+                                                   0x06020400u) & 0x3F3F3F3Fu;
+                B[1][c][k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, ho), __builtin_bit_cast(uint32_t, he),
+                                                   0x06020400u);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s.d[j] = h2f(r.d[j >> 1] >> (16 * (j & 1)));
+    }
+    static __device__ __forceinline__ float step(float acc, float xd, const Scale& s, int j, int isum, float) {
+        return __builtin_fmaf(xd, s.d[j] * static_cast<float>(isum), acc);
+    }
+};
+
+// Q8_0: w[b] holds values 8 G .. 8 G + 7 of row i's block b (32 values), dw the rows 4 G + j's eight f16 scales.
+template <>
+struct GemmTile<7> {
+    struct Raw {
+        u32x2 w[8];
+        u32x4 dw[4];
+    };
+    static __device__ __forceinline__ Raw load(const uint8_t* t, int lane) {
+        const int i = lane & 15, G = lane >> 4;
+        Raw r;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            r.w[b] = *reinterpret_cast<const u32x2*>(t + 256 + (64 * (2 * (b & 1) + (G >> 1)) + i + 16 * (b >> 1)) * 16 +
+                                                     8 * (G & 1));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r.dw[j] = *reinterpret_cast<const u32x4*>(t + 16 * (4 * G + j));
+        return r;
+    }
+    // the tile's term of (row 4 G + j, token) from the blocks' integer dots and the token's block scales
+    static __device__ __forceinline__ float tile_term(const Raw& r, int j, const i32x4 (&A)[8], const float (&xd)[8]) {
+        float p[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t dw = r.dw[j][q];
+            p[q] = pair_sum(q8_term32(xd[2 * q], h2f(dw), A[2 * q][j]), q8_term32(xd[2 * q + 1], h2f(dw >> 16), A[2 * q + 1][j]));
+        }
+        return tile_total(p[0], p[1], p[2], p[3]);
+    }
+};
+
+// Copies 16 bytes per lane from base + off to LDS at lds + 16 * lane (lds is wave-uniform), past the
+// registers. The compiler does not count these loads: lds_dma_wait before the barrier that publishes them.
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+template <uint32_t TYPE, int TP, int OCC>
+__global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a, int32_t n_rg) {
+    constexpr int NW = kGemmWaves, NTHR = NW * kWave, NTOK = 16 * TP, NROW = 16 * NW;
+    constexpr bool Q8 = TYPE == 7, PIPE = OCC < 4;
+    constexpr uint32_t TB = tile_bytes(TYPE);
+    constexpr int CPW = NTOK / (4 * NW);  // 1 KB copies (four token rows) per wave of a staged tile
+    static_assert(NTOK % (4 * NW) == 0 && 2 * NTOK <= NTHR, "whole copies per wave, half a token's sums per thread");
+    constexpr int VSTRIDE = NROW + 1;  // epilogue row stride (floats)
+    constexpr int CODES = 2 * NTOK * 256, VALS = NTOK * VSTRIDE * 4;
+    constexpr int SIDE = Q8 ? 8 : 1;  // scales per token and tile
+    __shared__ __align__(16) uint8_t codes[CODES > VALS ? CODES : VALS];  // then the epilogue's values
+    __shared__ __align__(16) f16x8 sums[2][Q8 ? 1 : 2 * NTOK];            // the tile's sixteen 16-value code sums
+    __shared__ __align__(16) float scales[2][NTOK * SIDE];
+    using T = GemmTile<TYPE>;
+    const int n_tok = a.n_tok, n_grp = ((n_tok + 15) / 16 + TP - 1) / TP;
+    const int n_sets = (n_rg + NW - 1) / NW;
+    // work-group k runs on XCD k % 8; an XCD takes a contiguous share of the (row set, token group) list, token
+    // groups of one set in a row, so that they share the set's weights in its L2
+    const int total_wgs = n_sets * n_grp, share = (total_wgs + 7) / 8;
+    const int at = static_cast<int>(blockIdx.x & 7u) * share + static_cast<int>(blockIdx.x >> 3);
+    if (static_cast<int>(blockIdx.x >> 3) >= share || at >= total_wgs) return;
+    const int set = at / n_grp, t0 = (at - set * n_grp) * NTOK;
+    const int nt = min(NTOK, n_tok - t0);
+    const int K = static_cast<int>(a.mat.cols), nb = K / 256;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+    const int i = lane & 15, G = lane >> 4;
+    const Act8 xq = a.xq;
+    // a row group past the matrix repeats its last one (its rows are never stored)
+    const uint8_t* base = a.mat.data + static_cast<size_t>(min(set * NW + wave, n_rg - 1)) * nb * TB;
+
+    // Staging of a K tile: the codes are copied straight to LDS (copy c of the tile holds token rows 4 c .. 4 c + 3;
+    // 16-byte piece p of row r lies at slot p ^ (r % 16), so that sixteen rows' reads of one piece hit all banks),
+    // sums and scales pass through registers. Token rows past the step repeat its last row; element offsets are
+    // unsigned 32-bit.
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) uint8_t*) codes));
+    uint32_t src_off[CPW];
+#pragma unroll
+    for (int u = 0; u < CPW; ++u) {
+        const uint32_t row = 4u * (wave * CPW + u) + (lane >> 4), piece = (lane & 15) ^ (row & 15);
+        src_off[u] = static_cast<uint32_t>(min(t0 + static_cast<int>(row), n_tok - 1)) * static_cast<uint32_t>(K) + 16u * piece;
+    }
+    auto stage_codes = [&](int b, int buf) {
+#pragma unroll
+        for (int u = 0; u < CPW; ++u) {
+            lds_dma16(xq.q + 256 * b, src_off[u], lds0 + static_cast<uint32_t>(buf * NTOK * 256 + (wave * CPW + u) * 1024));
+        }
+    };
+    struct Stage {
+        u32x4 s;
+        float d;
+    };
+    const uint32_t half_tok = static_cast<uint32_t>(min(t0 + static_cast<int>(threadIdx.x >> 1), n_tok - 1));
+    const uint32_t one_tok = static_cast<uint32_t>(min(t0 + static_cast<int>(threadIdx.x), n_tok - 1));
+    auto stage_load = [&](int b) {
+        Stage st{};
+        if (threadIdx.x < 2 * NTOK) {  // half a token's sums, or (Q8_0) half its eight block scales
+            if constexpr (Q8) {
+                st.s = *reinterpret_cast<const u32x4*>(xq.d + (half_tok * static_cast<uint32_t>(K / 32) + 8u * b +
+                                                               4u * (threadIdx.x & 1)));
+            } else if constexpr (T::kMins) {
+                st.s = *reinterpret_cast<const u32x4*>(xq.s + (half_tok * static_cast<uint32_t>(K / 16) + 16u * b +
+                                                               8u * (threadIdx.x & 1)));
+            }
+        }
+        if (!Q8 && threadIdx.x < NTOK) st.d = xq.d[one_tok * static_cast<uint32_t>(nb) + b];
+        return st;
+    };
+    auto stage_store = [&](const Stage& st, int buf) {
+        if (threadIdx.x < 2 * NTOK) {
+            if constexpr (Q8) {
+                reinterpret_cast<u32x4*>(&scales[buf][0])[threadIdx.x] = st.s;
+            } else if constexpr (T::kMins) {
+                f16x8 h;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    h[2 * k] = static_cast<_Float16>(static_cast<int16_t>(st.s[k] & 0xFFFFu));
+                    h[2 * k + 1] = static_cast<_Float16>(static_cast<int16_t>(st.s[k] >> 16));
+                }
+                sums[buf][threadIdx.x] = h;
+            }
+        }
+        if (!Q8 && threadIdx.x < NTOK) scales[buf][threadIdx.x] = st.d;
+    };
+    // the tile after b in the decode waves' order
+    auto next_tile = [&](int b) { return b + 8 < nb ? b + 8 : (b & 7) + 1; };
+
+    float total[TP][4], chain[TP][4];
+#pragma unroll
+    for (int tl = 0; tl < TP; ++tl) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) total[tl][j] = chain[tl][j] = 0.0F;
+    }
+    stage_codes(0, 0);
+    stage_store(stage_load(0), 0);
+    typename T::Raw raw = T::load(base, lane);
+    // the lane's first code piece of a token row: 64 G (K-quants), 8 G (Q8_0); piece k beyond it: ^ 16 k, ^ 32 k
+    const uint32_t code_at = static_cast<uint32_t>(i) * 256u +
+                             (Q8 ? (((G >> 1) ^ i) << 4) + 8 * (G & 1) : ((4 * G) ^ i) << 4);
+    lds_dma_wait();
+    __syncthreads();
+    int b = 0;
+    for (int s = 0; s < nb; ++s) {
+        const int buf = s & 1;
+        const int bn = s + 1 < nb ? next_tile(b) : b;  // clamped: issued unconditionally
+        const Stage st = stage_load(bn);
+        if (s + 1 < nb) stage_codes(bn, buf ^ 1);
+        const uint8_t* tile_codes = &codes[buf * NTOK * 256];
+        if constexpr (Q8) {
+#pragma unroll
+            for (int tl = 0; tl < TP; ++tl) {
+                const f32x4* xs = reinterpret_cast<const f32x4*>(&scales[buf][8 * (16 * tl + i)]);
+                const f32x4 x0 = xs[0], x1 = xs[1];
+                const float xd[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+                i32x4 A[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    A[k] = mfma_i8(pack2(raw.w[k].x, raw.w[k].y),
+                                   *reinterpret_cast<const long*>(tile_codes + tl * 4096 + (code_at ^ (32u * k))));
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) chain[tl][j] += T::tile_term(raw, j, A, xd);
+            }
+            raw = T::load(base + static_cast<size_t>(bn) * TB, lane);
+        } else {
+            u32x4 B[T::kChains][4];
+            typename T::Scale sc;
+            if constexpr (!PIPE) raw = T::load(base + static_cast<size_t>(b) * TB, lane);
+            T::fold(raw, lane, B, sc);
+            // the next tile's weight loads stay here, a whole tile ahead of their use
+            if constexpr (PIPE) raw = T::load(base + static_cast<size_t>(bn) * TB, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            i32x4 av[2][4], D[2][T::kChains];
+            f32x4 ms[2];
+            f16x4 xs[2] = {};
+            auto read = [&](int tl) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    av[tl & 1][m] = *reinterpret_cast<const i32x4*>(tile_codes + tl * 4096 + (code_at ^ (16u * m)));
+                if constexpr (T::kMins) xs[tl & 1] = reinterpret_cast<const f16x4*>(&sums[buf][2 * (16 * tl + i)])[G];
+            };
+            auto product = [&](int tl) {
+                const int e = tl & 1;
+#pragma unroll
+                for (int c = 0; c < T::kChains; ++c) D[e][c] = i32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+#pragma unroll
+                    for (int c = 0; c < T::kChains; ++c) {
+                        D[e][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, B[c][m]), av[e][m],
+                                                                        D[e][c], 0, 0, 0);
+                    }
+                }
+                ms[e] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
+                if constexpr (T::kMins) ms[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(sc.mins, xs[e], ms[e], 0, 0, 0);
+            };
+            auto step = [&](int tl) {
+                const int e = tl & 1;
+                const float xdt = scales[buf][16 * tl + i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    int isum = D[e][0][j];
+                    if constexpr (T::kChains == 2) isum += static_cast<int>(static_cast<uint32_t>(D[e][1][j]) << T::kShift);
+                    chain[tl][j] = T::step(chain[tl][j], xdt, sc, j, isum, ms[e][j]);
+                }
+            };
+            if constexpr (!PIPE) {
+#pragma unroll
+                for (int tl = 0; tl < TP; ++tl) {
+                    read(tl);
+                    product(tl);
+                    step(tl);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                // the code reads of token tile tl + 1, the matrix products of tl and the float step of tl - 1 are
+                // independent and interleave
+                read(0);
+#pragma unroll
+                for (int tl = 0; tl < TP; ++tl) {
+                    if (tl + 1 < TP) read(tl + 1);
+                    product(tl);
+                    if (tl > 0) {
+                        step(tl - 1);
+                        constexpr int M = 4 * T::kChains + (T::kMins ? 1 : 0), V = (T::kChains == 2 ? 20 : 16) + 2;
+#pragma unroll
+                        for (int k = 0; k < M; ++k) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                       // one matrix product
+                            __builtin_amdgcn_sched_group_barrier(0x002, (V + M - 1) / M, 0);         // its share of the step
+                            if (k < 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);             // code reads of the next
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                step(TP - 1);
+            }
+        }
+        if (b + 8 >= nb) {
+            // the chain of tiles b mod 8 ends: its partial joins the total in wave order
+#pragma unroll
+            for (int tl = 0; tl < TP; ++tl) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    total[tl][j] += chain[tl][j];
+                    chain[tl][j] = 0.0F;
+                }
+            }
+        }
+        if (s + 1 < nb) stage_store(st, buf ^ 1);
+        b = bn;
+        lds_dma_wait();
+        __syncthreads();
+    }
+    // the staging buffers are free (the loop ends on a barrier): rows and tokens to the epilogue
+    float* vals = reinterpret_cast<float*>(&codes[0]);
+#pragma unroll
+    for (int tl = 0; tl < TP; ++tl) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vals[(16 * tl + i) * VSTRIDE + 16 * wave + 4 * G + j] = total[tl][j];
+    }
+    __syncthreads();
+    const int row0 = set * NROW, nrows = min(NROW, static_cast<int>(a.mat.rows) - row0);
+    const GemvArgs out = token_slice(a, t0, nt);
+    auto value = [&](int j, int tk) { return vals[tk * VSTRIDE + j]; };
+    // whole sets divide by a constant
+    if (nrows == NROW) gemv_epilogue<NTHR, kNoLogits>(out, row0, NROW, value, nullptr);
+    else gemv_epilogue<NTHR, kNoLogits>(out, row0, nrows, value, nullptr);
+}
+
+// The folded tiles for steps whose grid is too small for the long-step matmul: the decode matmul's eight waves (wave
+// w takes the K tiles w, w + 8, ...), R consecutive row groups and one 16-token tile per work-group. A wave loads its
+// K tile's activations (lane (i, G): token i's bytes 64 G .. 64 G + 63, its code sums and scales) once and runs them
+// against the R row groups' folded weight operands, the next weight tile in flight while one runs; no LDS and no
+// barrier until the waves' partials are summed in wave order, so every row equals the decode row bit for bit.
+template <uint32_t TYPE, int R>
+__global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg) {
     constexpr int W = kMmWaves;
-    constexpr uint32_t TB = tile_bytes(11);
-    constexpr uint32_t M4 = 0x0F0F0F0Fu;
+    constexpr bool Q8 = TYPE == 7;
+    constexpr uint32_t TB = tile_bytes(TYPE);
+    using T = GemmTile<TYPE>;
     __shared__ float red[W][16][16 * R];  // [wave][token][row]
     __shared__ float vals[16][16 * R];
     const int n_tok = a.n_tok, n_tt = (n_tok + 15) / 16;
@@ -2460,83 +2775,74 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_wide_q4r(GemvArgs a, int32_t 
     // the lane's token (rows past the step repeat its last row; never stored)
     const uint32_t tok = static_cast<uint32_t>(min(t0 + i, n_tok - 1));
     const uint8_t* base = a.mat.data + static_cast<size_t>(rg0) * nb * TB;
-    struct Raw {
-        uint32_t dd[4];
-        uint2 fw;
-        u32x4 w0, w1;
-    };
-    auto load_raw = [&](int rr, int b) {
-        const uint8_t* t = base + (static_cast<size_t>(rr) * nb + b) * TB;
-        Raw r;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r.dd[j] = *reinterpret_cast<const uint32_t*>(t + 16 * (4 * G + j));
-        r.fw = *reinterpret_cast<const uint2*>(t + 16 * i + 4 + 4 * ((3 * G) >> 2));
-        r.w0 = *reinterpret_cast<const u32x4*>(t + 256 + 16 * lane);
-        r.w1 = *reinterpret_cast<const u32x4*>(t + 1280 + 16 * lane);
-        return r;
-    };
-    auto sub_sum = [](uint32_t w) {
-        return static_cast<float>(static_cast<int16_t>(w & 0xFFFFu) + (static_cast<int32_t>(w) >> 16));
-    };
+    auto load_raw = [&](int rr, int b) { return T::load(base + (static_cast<size_t>(rr) * nb + b) * TB, lane); };
     float acc[R][4];
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[rr][j] = 0.0F;
     }
-    Raw cur = load_raw(0, min(wave, nb - 1));
+    typename T::Raw cur = load_raw(0, min(wave, nb - 1));
     for (int b = wave; b < nb; b += W) {
-        const u32x4* src = reinterpret_cast<const u32x4*>(xq.q + (tok * static_cast<uint32_t>(K) + 256u * b + 64u * G));
-        u32x4 xa[4];
+        const uint4* src = reinterpret_cast<const uint4*>(xq.q + (tok * static_cast<uint32_t>(K) + 256u * b + 64u * G));
+        uint4 xa[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) xa[m] = src[m];
-        const uint2 sw = *reinterpret_cast<const uint2*>(xq.s + (tok * static_cast<uint32_t>(K / 16) + 16u * b + 4u * G));
-        const float xd = xq.d[tok * static_cast<uint32_t>(nb) + b];
+        f16x4 xs = {};
+        float xd[Q8 ? 8 : 1];
+        long av[8];
+        if constexpr (Q8) {
+            const f32x4* ds = reinterpret_cast<const f32x4*>(xq.d + (tok * static_cast<uint32_t>(K / 32) + 8u * b));
+            const f32x4 d0 = ds[0], d1 = ds[1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                xd[k] = d0[k];
+                xd[4 + k] = d1[k];
+            }
+            wide_a_operands(xa, av);
+        } else {
+            xd[0] = xq.d[tok * static_cast<uint32_t>(nb) + b];
+            if constexpr (T::kMins) {
+                const uint2 sw = *reinterpret_cast<const uint2*>(xq.s + (tok * static_cast<uint32_t>(K / 16) + 16u * b + 4u * G));
+                xs = f16x4{static_cast<_Float16>(static_cast<int16_t>(sw.x & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.x >> 16)),
+                           static_cast<_Float16>(static_cast<int16_t>(sw.y & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.y >> 16))};
+            }
+        }
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
             // the next weight tile (the next row group's, else the wave's next K tile's first; clamped)
-            const Raw nxt = rr + 1 < nrg ? load_raw(rr + 1, b) : load_raw(0, min(b + W, nb - 1));
+            const typename T::Raw nxt = rr + 1 < nrg ? load_raw(rr + 1, b) : load_raw(0, min(b + W, nb - 1));
             if (rr < nrg) {
-                float d[4], dmin[4];  // rows 4 G + j
+                if constexpr (Q8) {
+                    i32x4 A[8];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    d[j] = h2f(cur.dd[j]);
-                    dmin[j] = h2f(cur.dd[j] >> 16);
-                }
-                // lane group G's 24-bit field of row i: sc 2G | sc 2G+1 | m 2G | m 2G+1
-                const uint32_t f = __builtin_amdgcn_alignbyte(cur.fw.y, cur.fw.x, (3 * G) & 3);
-                const uint32_t sca = f & 63u, scb = (f >> 6) & 63u;
-                const float ma = static_cast<float>((f >> 12) & 63u), mb = static_cast<float>((f >> 18) & 63u);
-                const u16x2 la = {static_cast<uint16_t>(sca & 7u), static_cast<uint16_t>(sca & 7u)};
-                const u16x2 ha = {static_cast<uint16_t>(sca >> 3), static_cast<uint16_t>(sca >> 3)};
-                const u16x2 lb = {static_cast<uint16_t>(scb & 7u), static_cast<uint16_t>(scb & 7u)};
-                const u16x2 hb = {static_cast<uint16_t>(scb >> 3), static_cast<uint16_t>(scb >> 3)};
-                auto fold = [](uint32_t c, u16x2 sv) {
-                    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, c) * sv);
-                };
-                i32x4 DL = {0, 0, 0, 0}, DH = {0, 0, 0, 0};
+                    for (int k = 0; k < 8; ++k) A[k] = mfma_i8(pack2(cur.w[k].x, cur.w[k].y), av[k]);
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const u32x4 w = m & 1 ? cur.w1 : cur.w0;
-                    const u16x2 sl = m < 2 ? la : lb, sh = m < 2 ? ha : hb;
-                    u32x4 bl, bh;
+                    for (int j = 0; j < 4; ++j) acc[rr][j] += T::tile_term(cur, j, A, xd);
+                } else {
+                    u32x4 B[T::kChains][4];
+                    typename T::Scale sc;
+                    T::fold(cur, lane, B, sc);
+                    i32x4 D[T::kChains];
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t c = m < 2 ? w[k] & M4 : (w[k] >> 4) & M4;
-                        bl[k] = fold(c, sl);
-                        bh[k] = fold(c, sh);
+                    for (int c = 0; c < T::kChains; ++c) D[c] = i32x4{0, 0, 0, 0};
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+#pragma unroll
+                        for (int c = 0; c < T::kChains; ++c) {
+                            D[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, B[c][m]),
+                                                                         __builtin_bit_cast(i32x4, xa[m]), D[c], 0, 0, 0);
+                        }
                     }
-                    const i32x4 av = __builtin_bit_cast(i32x4, xa[m]);
-                    DL = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, bl), av, DL, 0, 0, 0);
-                    DH = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, bh), av, DH, 0, 0, 0);
-                }
-                // token i's 32-value code sums of sub-blocks 2G, 2G + 1
-                f32x4 ms = {0.0F, 0.0F, 0.0F, 0.0F};
-                ms = __builtin_amdgcn_mfma_f32_16x16x4f32(ma, sub_sum(sw.x), ms, 0, 0, 0);
-                ms = __builtin_amdgcn_mfma_f32_16x16x4f32(mb, sub_sum(sw.y), ms, 0, 0, 0);
+                    f32x4 ms = {0.0F, 0.0F, 0.0F, 0.0F};
+                    if constexpr (T::kMins) ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sc.mins, xs, ms, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[rr][j] = q4k_term_f(acc[rr][j], xd, d[j], dmin[j], DL[j] + 8 * DH[j], ms[j]);
+                    for (int j = 0; j < 4; ++j) {
+                        int isum = D[0][j];
+                        if constexpr (T::kChains == 2) isum += static_cast<int>(static_cast<uint32_t>(D[1][j]) << T::kShift);
+                        acc[rr][j] = T::step(acc[rr][j], xd[0], sc, j, isum, ms[j]);
+                    }
+                }
             }
             cur = nxt;
         }
@@ -3156,6 +3462,211 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention_mfma(const float* __
     }
 }
 
+// Causal attention of a prefill chunk (one sequence, many rows): no key splits and no merge. Work-group =
+// (kv head, 64 RQ of its G x rows query rows), each wave 16 RQ of them; the work-group walks the keys in blocks of 64
+// that all four waves read from LDS (copied there directly, the next block in flight while one is multiplied), so a
+// key and value byte is fetched once per 64 RQ query rows instead of once per 16. The fragments are
+// k_attention_mfma's: S^T = K . Q^T with the queries as f16 hi + lo, O^T += V^T . P^T with the probabilities as f16
+// hi + lo; P . V runs on 16x16x32 products whose 32 key slots are lane group grp's keys 4 grp .. + 3 of two 16-key
+// tiles, as the S^T fragments hold them. Work-groups with the longest key ranges start first.
+// LDS: K row r's 16-byte piece p lies at slot p ^ (r % 16) (head dim 64: p ^ (r / 2 % 8)), V tiles as in the cache.
+constexpr int kPrefillAttnKeys = 64;
+
+__device__ __forceinline__ float lane_group_max(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+__device__ __forceinline__ float lane_group_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+template <int HD, int RQ>
+__global__ __launch_bounds__(kAttnThreads, 2) void k_attention_prefill(const float* __restrict__ q,
+                                                                       const StepDev* __restrict__ step, int32_t layer,
+                                                                       int32_t n_head, int32_t n_head_kv,
+                                                                       float* __restrict__ out) {
+    constexpr int W = kAttnThreads / kWave, KS = HD / 32, DB = HD / 16, R = kAttnRows, KB = kPrefillAttnKeys;
+    constexpr int PPR = HD / 8;              // 16-byte pieces of a K row
+    constexpr int KPC = kWave / PPR;         // K rows per 1 KB copy
+    constexpr int BLOCK = KB * HD * 2;       // bytes of a block's K, and of its V
+    constexpr int CPW = BLOCK / 1024 / W;    // copies per wave
+    __shared__ __align__(16) uint8_t kv[2][2][BLOCK];
+    const int32_t pos0 = step->seqs[0].pos0, len = step->seqs[0].len, row0 = step->seqs[0].row0;
+    const int32_t capacity = step->seqs[0].capacity;
+    const int G = n_head / n_head_kv, NQ = G * len, H = n_head * HD, kvh = blockIdx.y;
+    const int q_begin = static_cast<int>(gridDim.x - 1 - blockIdx.x) * W * R * RQ;
+    if (q_begin >= NQ) return;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+    const int r = lane & (R - 1), grp = lane >> 4;
+    const size_t head_base = (static_cast<size_t>(layer) * n_head_kv + kvh) * capacity * HD;
+    const uint16_t* kc = step->seqs[0].k + head_base;
+    const uint16_t* vt = step->seqs[0].v + head_base;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) uint8_t*) &kv[0][0][0]));
+    // keys of the work-group: up to its last query row's position
+    const int n_keys = pos0 + min(NQ - 1, q_begin + W * R * RQ - 1) / G + 1;
+    const int n_blocks = (n_keys + KB - 1) / KB;
+    // capacity is a multiple of 16, so a clamped 16-key tile keeps all its keys in bounds (its keys are masked)
+    auto stage = [&](int kb, int buf) {
+        const uint32_t at = lds0 + static_cast<uint32_t>(buf * 2 * BLOCK);
+#pragma unroll
+        for (int u = 0; u < CPW; ++u) {
+            const int c = wave * CPW + u;
+            const int key = c * KPC + lane / PPR;
+            const int piece = (lane % PPR) ^ (HD == 128 ? key & 15 : (key >> 1) & 7);
+            const int t = min(kb * KB + (key & ~15), capacity - R) + (key & 15);
+            lds_dma16(kc, static_cast<uint32_t>(t * HD * 2 + 16 * piece), at + static_cast<uint32_t>(c * 1024));
+            const int tile = c / (HD / 32), part = c % (HD / 32);
+            const int tv = min(kb * KB + tile * R, capacity - R);
+            lds_dma16(vt, static_cast<uint32_t>(tv * HD * 2 + part * 1024 + 16 * lane),
+                      at + static_cast<uint32_t>(BLOCK + c * 1024));
+        }
+    };
+    stage(0, 0);
+
+    // B operands of S^T: row r of each row group, dims 32 s + 8 grp .. + 7, as f16 hi + lo
+    int limit[RQ];  // last visible key of the lane's row (causal; -1: no row)
+    h8 qhi[RQ][KS], qlo[RQ][KS];
+    const float scale = 1.0F / sqrtf(static_cast<float>(HD));
+#pragma unroll
+    for (int g = 0; g < RQ; ++g) {
+        const int qr = q_begin + (wave * RQ + g) * R + r, qi = min(qr, NQ - 1);
+        const bool row_ok = qr < NQ;
+        const int tr = qi / G, head = kvh * G + qi % G;
+        limit[g] = row_ok ? pos0 + tr : -1;
+        const float* qrow = q + static_cast<size_t>(row0 + tr) * H + head * HD + 8 * grp;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const float4 a = *reinterpret_cast<const float4*>(qrow + 32 * s);
+            const float4 b = *reinterpret_cast<const float4*>(qrow + 32 * s + 4);
+            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float v = row_ok ? x[j] * scale : 0.0F;
+                qhi[g][s][j] = static_cast<_Float16>(v);
+                qlo[g][s][j] = static_cast<_Float16>(v - static_cast<float>(qhi[g][s][j]));
+            }
+        }
+    }
+    const int first_limit = pos0 + q_begin / G;  // smallest causal bound of the work-group's rows
+    const bool whole = q_begin + W * R * RQ <= NQ;
+    float m[RQ], l[RQ];
+    f32x4 o[RQ][DB];
+#pragma unroll
+    for (int g = 0; g < RQ; ++g) {
+        m[g] = -INFINITY;
+        l[g] = 0.0F;
+#pragma unroll
+        for (int d = 0; d < DB; ++d) o[g][d] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
+    }
+    lds_dma_wait();
+    __syncthreads();
+    for (int kb = 0; kb < n_blocks; ++kb) {
+        const int buf = kb & 1;
+        if (kb + 1 < n_blocks) stage(kb + 1, buf ^ 1);
+        const uint8_t* kt = &kv[buf][0][0];
+        const uint8_t* vl = &kv[buf][1][0];
+        f32x4 sc[RQ][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int key = 16 * t + r, sw = HD == 128 ? key & 15 : (key >> 1) & 7;
+#pragma unroll
+            for (int g = 0; g < RQ; ++g) sc[g][t] = f32x4{0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const h8 ka = *reinterpret_cast<const h8*>(kt + key * (HD * 2) + 16 * ((4 * s + grp) ^ sw));
+#pragma unroll
+                for (int g = 0; g < RQ; ++g) {
+                    sc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi[g][s], sc[g][t], 0, 0, 0);
+                    sc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo[g][s], sc[g][t], 0, 0, 0);
+                }
+            }
+        }
+        if (!whole || kb * KB + KB - 1 > first_limit) {
+#pragma unroll
+            for (int g = 0; g < RQ; ++g) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if (kb * KB + 16 * t + 4 * grp + j > limit[g]) sc[g][t][j] = -INFINITY;
+                    }
+                }
+            }
+        }
+        h8 phi[RQ][2], plo[RQ][2];
+#pragma unroll
+        for (int g = 0; g < RQ; ++g) {
+            float tmax = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) tmax = fmaxf(tmax, sc[g][t][j]);
+            }
+            const float m_new = fmaxf(m[g], lane_group_max(tmax));
+            const float base = m_new == -INFINITY ? 0.0F : m_new;  // a row without a visible key keeps zeros
+            float sum = 0.0F;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                float p[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    p[j] = expf(sc[g][t][j] - base);
+                    const _Float16 hi = static_cast<_Float16>(p[j]);
+                    phi[g][t >> 1][4 * (t & 1) + j] = hi;
+                    plo[g][t >> 1][4 * (t & 1) + j] = static_cast<_Float16>(p[j] - static_cast<float>(hi));
+                }
+                sum += (p[0] + p[1]) + (p[2] + p[3]);
+            }
+            // the running output is rescaled only when some row of the group has a new maximum
+            if (__any(m_new != m[g])) {
+                const float alpha = expf(m[g] - base);
+                l[g] *= alpha;
+#pragma unroll
+                for (int d = 0; d < DB; ++d) o[g][d] *= alpha;
+            }
+            l[g] += sum;
+            m[g] = m_new;
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const uint8_t* vp = vl + 2 * u * (R * HD * 2) + (16 * d + r) * 32 + 8 * grp;
+                const h4 v0 = *reinterpret_cast<const h4*>(vp), v1 = *reinterpret_cast<const h4*>(vp + R * HD * 2);
+                const h8 va = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int g = 0; g < RQ; ++g) {
+                    o[g][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, phi[g][u], o[g][d], 0, 0, 0);
+                    o[g][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, plo[g][u], o[g][d], 0, 0, 0);
+                }
+            }
+        }
+        lds_dma_wait();
+        __syncthreads();
+    }
+#pragma unroll
+    for (int g = 0; g < RQ; ++g) {
+        const float total = lane_group_sum(l[g]);
+        const int qr = q_begin + (wave * RQ + g) * R + r;
+        if (qr < NQ) {
+            float* dst = out + static_cast<size_t>(row0 + qr / G) * H + (kvh * G + qr % G) * HD + 4 * grp;
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                *reinterpret_cast<f32x4*>(dst + 16 * d) =
+                    f32x4{o[g][d][0] / total, o[g][d][1] / total, o[g][d][2] / total, o[g][d][3] / total};
+            }
+        }
+    }
+}
+
 // Combines the split partials of every (row, head): one work-group per
 // (row, 256 output values); with xq set the 256 values are quantized into xq.
 // Every split slot below n_slots (the attention grid's splits) holds this
@@ -3244,7 +3755,7 @@ __global__ void k_finish(unsigned long long* best, const StepDev* step, int32_t 
         bool open = true;
         for (int i = 0; i < n_out; ++i) {
             const int r = step->out_row[i];
-            if (step->seq[r] != s || !open) continue;
+            if (step->rows[r].seq != s || !open) continue;
             bool end = false;
             for (int e = 0; e < n_end; ++e) end |= tok[i] == step->end_token[e];
             if (step->draft[i] >= 0 && tok[i] == step->draft[i] && !end) ++accepted;
@@ -3560,7 +4071,6 @@ void launch_quantize_norm(const float* x, int32_t stride, const int32_t* gather,
 }
 
 constexpr int kWideMinWgs = 512;
-constexpr int kWideRgMinWgs = 256;  // one work-group per CU
 constexpr int kWideLogitsWgs = 1024;
 constexpr int kWideQ4kWaves = 4;
 constexpr int kWideQ4kMinWgs = 256;
@@ -3581,6 +4091,52 @@ int32_t wide_min_rows(uint32_t type) {
     }
 }
 
+// Which kernel a layer matrix's step takes, by the work-groups that 64 rows x 16 TP tokens make of it (256 CUs;
+// measured over 9..2048 rows on matrices of 1536..55296 rows). Each K tile costs a wave of the long-step matmul about
+// 1 us of latency however few tokens it carries, so below about 1.5 work-groups per CU the K-split kernel is faster
+// (7B Q4_K down, 56 row sets: 160 rows 79 us against 83, 256 rows 109 against 86), unless K is so short that its
+// eight waves have no two tiles each (2048 x 1536 Q6_K, 256 rows: 12.7 against 10.4).
+constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192;
+constexpr int kGemmFillWgs = 1024;  // four waves per SIMD everywhere
+constexpr int kGemmShortTiles = 8;
+
+template <uint32_t TYPE, int TP, int OCC>
+void gemm(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
+    const int wgs = (n_rg + kGemmWaves - 1) / kGemmWaves * ((n_tt + TP - 1) / TP);
+    launch(k_mm_gemm<TYPE, TP, OCC>, dim3((wgs + 7) / 8 * 8), dim3(kGemmWaves * kWave), 0, stream, a, n_rg);
+}
+
+template <uint32_t TYPE, int R>
+void fold(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
+    launch(k_mm_fold<TYPE, R>, dim3(((n_rg + R - 1) / R + 7) / 8 * 8 * n_tt), dim3(kMmThreads), 0, stream, a, n_rg);
+}
+
+// A K-quant layer matrix.
+template <uint32_t TYPE>
+void folded(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
+    const int n_sets = (n_rg + kGemmWaves - 1) / kGemmWaves;
+    auto wgs = [&](int tp) { return n_sets * ((n_tt + tp - 1) / tp); };
+    const bool short_k = static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles;
+    if constexpr (TYPE == 11) {
+        // one or two token tiles against many row groups stream the weights from HBM
+        if (n_tt <= 2 && n_sets >= kWideQ4kMinWgs) {
+            const dim3 g((n_sets + 7) / 8 * 8), b(kWideQ4kWaves * kWave);
+            if (n_tt == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg, 2);
+            else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg, 1);
+            check(hipGetLastError(), "wide matmul launch");
+            return;
+        }
+    }
+    if (n_tt >= 3 && wgs(4) >= kGemmFillWgs) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
+    else if (n_tt >= 16 && wgs(8) >= kGemmMinWgs) gemm<TYPE, 8, 2>(a, n_rg, n_tt, stream);
+    else if (n_tt >= 3 && wgs(4) >= kGemmMinWgs) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
+    else if (n_tt >= 2 && wgs(2) >= (short_k ? kGemmShortWgs : kGemmMinWgs)) gemm<TYPE, 2, 3>(a, n_rg, n_tt, stream);
+    // one row group per work-group only while that is at most a work-group per CU
+    else if (n_rg * n_tt <= 256) fold<TYPE, 1>(a, n_rg, n_tt, stream);
+    else fold<TYPE, 2>(a, n_rg, n_tt, stream);
+    check(hipGetLastError(), "wide matmul launch");
+}
+
 void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
     if (!wide_matmul_supported(a_in.mat.type) || a_in.xq.q == nullptr || a_in.xq.K != static_cast<int32_t>(a_in.mat.cols) ||
         a_in.mat.cols % kActBlock != 0 || a_in.n_tok < 1 || a_in.n_tok > kWideRows) {
@@ -3593,55 +4149,25 @@ void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
     mm_a32(a_in);  // validates the activation block for the weight type
     const GemvArgs& a = a_in;
     const int n_rg = (static_cast<int>(a.mat.rows) + 15) / 16, n_tt = (a.n_tok + 15) / 16;
+    const bool merged = a.mode == kLogits;  // the head kernel: the only one with the argmax epilogue
+    if (!merged && a.mat.type != 7) {
+        if (a.mat.type == 9) folded<9>(a, n_rg, n_tt, stream);
+        else if (a.mat.type == 11) folded<11>(a, n_rg, n_tt, stream);
+        else folded<13>(a, n_rg, n_tt, stream);
+        return;
+    }
+    if (!merged && n_tt >= 2) {
+        // Q8_0, bound by its float step per 32-value block: one tile shape
+        const int wgs = (n_rg + kGemmWaves - 1) / kGemmWaves * ((n_tt + 1) / 2);
+        if (wgs >= (static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs)) {
+            gemm<7, 2, 3>(a, n_rg, n_tt, stream);
+            check(hipGetLastError(), "wide matmul launch");
+            return;
+        }
+    }
     // as many token tiles per work-group as still leave kWideMinWgs work-groups
     int tpw = min(n_tt, kWideTpw);
     while (tpw > 1 && n_rg * ((n_tt + tpw - 1) / tpw) < kWideMinWgs) --tpw;
-    const bool merged = a.mode == kLogits;  // the head kernel: the only one with the argmax epilogue
-    if (a.mat.type == 11 && !merged) {
-        // Q4_K matrices with many row groups: whole-K waves over all of the
-        // step's token tiles, while that still leaves kWideQ4kMinWgs work-groups
-        const int n_sets = (n_rg + kWideQ4kWaves - 1) / kWideQ4kWaves;
-        if (n_sets >= kWideQ4kMinWgs) {
-            // up to four token tiles per work-group; longer steps run as several token groups
-            const int tpw4 = min(n_tt, 4), n_grp4 = (n_tt + tpw4 - 1) / tpw4;
-            const dim3 g((n_sets + 7) / 8 * 8 * n_grp4), b(kWideQ4kWaves * kWave);
-            if (tpw4 > 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 4>, g, b, 0, stream, a, n_rg, tpw4);
-            else if (tpw4 == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg, tpw4);
-            else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg, tpw4);
-            check(hipGetLastError(), "wide matmul launch");
-            return;
-        }
-        // fewer row groups: two row groups and one token tile per work-group, the decode
-        // waves' K split, while one work-group per CU remains
-        if ((n_rg + 1) / 2 * n_tt >= kWideRgMinWgs) {
-            const dim3 g(((n_rg + 1) / 2 + 7) / 8 * 8 * n_tt), b(kMmThreads);
-            launch(k_mm_wide_q4r<2>, g, b, 0, stream, a, n_rg);
-            check(hipGetLastError(), "wide matmul launch");
-            return;
-        }
-    }
-    // K-quant layer matrices: one token tile and several row groups per work-group, every
-    // activation load shared by the row groups: four (Q4_K only: the other formats'
-    // operands take the registers) while kWideMinWgs work-groups remain, else two while
-    // one work-group per CU remains (Q6_K and Q2_K matrices, and Q4_K ones too small for
-    // the folded-scale kernels above)
-    int rgs = 1;
-    if (!merged && a.mat.type != 7) {
-        if (a.mat.type == 11 && (n_rg + 3) / 4 * n_tt >= kWideMinWgs) rgs = 4;
-        else if ((n_rg + 1) / 2 * n_tt >= kWideRgMinWgs) rgs = 2;
-    }
-    if (rgs > 1) {
-        const int tp1 = 1;
-        const dim3 g(((n_rg + rgs - 1) / rgs + 7) / 8 * 8 * n_tt), b(kMmThreads);
-        switch (a.mat.type * 8 + rgs) {
-        case 11 * 8 + 4: launch(k_mm_wide_rg<11, 4, 1, false>, g, b, 0, stream, a, n_rg, tp1); break;
-        case 11 * 8 + 2: launch(k_mm_wide_rg<11, 2, 1, false>, g, b, 0, stream, a, n_rg, tp1); break;
-        case 13 * 8 + 2: launch(k_mm_wide_rg<13, 2, 1, false>, g, b, 0, stream, a, n_rg, tp1); break;
-        default: launch(k_mm_wide_rg<9, 2, 1, false>, g, b, 0, stream, a, n_rg, tp1); break;
-        }
-        check(hipGetLastError(), "wide matmul launch");
-        return;
-    }
     // the head: row groups per work-group so that about kWideLogitsWgs work-groups merge their argmax
     const int rpw = a.mode == kLogits ? std::max(1, n_rg / kWideLogitsWgs) : 1;
     const int grid = (n_rg + 8 * rpw - 1) / (8 * rpw) * 8 * ((n_tt + tpw - 1) / tpw);
@@ -3674,6 +4200,9 @@ void launch_embed(const DMat& table, const StepDev* step, float* h, int32_t n_ro
     launch(k_embed, grid, dim3(256), 0, stream, table, step, h, H, best, n_best);
     check(hipGetLastError(), "embed launch");
 }
+
+// Fewest work-groups of 64 query rows from which a prefill chunk runs without key splits.
+constexpr int kPrefillAttnMinWgs = 128;
 
 int32_t attention_max_rows(int32_t head_dim) {
     // the matrix-core kernel takes any number of 16-row groups; the generic one up to kMaxAttnQGroups groups of 8
@@ -3734,6 +4263,31 @@ void launch_attention(const float* q, const StepDev* step, int32_t max_len, int3
                partial);
     }
     check(hipGetLastError(), "attention launch");
+}
+
+bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim) {
+    if (n_seq != 1 || n_rows <= kQuadGroupRows || (head_dim != 128 && head_dim != 64)) return false;
+    const int qblocks = (n_head / n_head_kv * n_rows + 4 * kAttnRows - 1) / (4 * kAttnRows);
+    return n_rows > kMaxRows || qblocks * n_head_kv >= kPrefillAttnMinWgs;
+}
+
+void launch_attention_prefill(const float* q, const StepDev* step, int32_t n_rows, int32_t layer, int32_t n_head,
+                              int32_t n_head_kv, int32_t head_dim, float* out, hipStream_t stream) {
+    if (head_dim != 128 && head_dim != 64) throw std::invalid_argument("prefill attention supports head dims 64 and 128");
+    const int NQ = n_head / n_head_kv * n_rows, per = 4 * kAttnRows;
+    // two row groups per wave where that leaves a work-group per resident slot
+    const int wide = (NQ + 2 * per - 1) / (2 * per);
+    const bool two = wide * n_head_kv >= kAttnResidentWgs;
+    const dim3 grid(two ? wide : (NQ + per - 1) / per, n_head_kv), block(kAttnThreads);
+    auto go = [&](auto kernel) { launch(kernel, grid, block, 0, stream, q, step, layer, n_head, n_head_kv, out); };
+    if (head_dim == 128) {
+        if (two) go(k_attention_prefill<128, 2>);
+        else go(k_attention_prefill<128, 1>);
+    } else {
+        if (two) go(k_attention_prefill<64, 2>);
+        else go(k_attention_prefill<64, 1>);
+    }
+    check(hipGetLastError(), "prefill attention launch");
 }
 
 void launch_attention_merge(const float* partial, const StepDev* step, int32_t n_rows, int32_t n_head,

@@ -10,12 +10,15 @@
 
 namespace jfh::gpu {
 
-// Token rows of one step (a prefill chunk is at most this long).
+// Token rows of one step (sum over sequences).
 constexpr int kMaxRows = 256;
+// Token rows of one prefill chunk: long enough that the layer matrices fill the chip with work-groups of 64 rows x
+// 128 tokens and their weights are read once per 2048 tokens.
+constexpr int kPrefillRows = 2048;
 // Token groups of at least this many rows (int8 or RMS-normalized input) of
 // the quantized formats (Q4_K, Q6_K, Q8_0, Q2_K) run as token quads on matrix
 // cores.
-constexpr int kQuadMinRows = 2;        // token rows of one step (sum over sequences)
+constexpr int kQuadMinRows = 2;
 // Token rows per matrix-core launch of the token-quad matmul (longer steps
 // run in groups of this many rows).
 constexpr int kQuadGroupRows = 16;
@@ -83,19 +86,24 @@ struct SeqDev {
     int32_t pos0;    // position of its first row
 };
 
+// One token row of a step.
+struct RowDev {
+    int32_t token;
+    int32_t pos;
+    int32_t seq;
+};
+
 // Step description in device memory, rewritten before every launch sequence.
 struct StepDev {
     int32_t n_rows;
     int32_t n_seq;
     int32_t n_out;                 // rows that produce logits
     int32_t n_end;                 // end-of-generation ids in end_token
-    int32_t token[kMaxRows];
-    int32_t pos[kMaxRows];
-    int32_t seq[kMaxRows];
     int32_t out_row[kMaxRows];     // step row of each logits row
     int32_t draft[kMaxRows];       // token the logits row is compared with (-1: none)
     int32_t end_token[kMaxEndTokens];
     SeqDev seqs[kMaxSeq];
+    RowDev rows[kPrefillRows];     // last: a step uploads the rows it has
 };
 
 // Result block copied back to the host after a step.
@@ -175,7 +183,7 @@ void launch_quantize_norm(const float* x, int32_t stride, const int32_t* gather,
                           int32_t n_rows, const Act8& out, hipStream_t stream);
 // Token rows of one matrix-core matmul launch (steps with more rows than the
 // decode matmul's 8-row groups).
-constexpr int kWideRows = kMaxRows;
+constexpr int kWideRows = kPrefillRows;
 // Whether launch_gemv_wide takes matrices of this type.
 bool wide_matmul_supported(uint32_t type);
 // Fewest token rows from which launch_gemv_wide outruns the token-quad
@@ -194,6 +202,12 @@ void launch_gemv_wide(const GemvArgs& a, hipStream_t stream);
 void launch_attention(const float* q, const StepDev* step, int32_t max_len, int32_t n_seq, int32_t layer,
                       int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t splits, float* partial,
                       hipStream_t stream, int32_t slots = 0);
+// Attention of one sequence's n_rows rows (a prefill chunk; head dims 64 and 128) without key splits: writes the
+// attention output rows to out [row][n_head * head_dim]. attention_prefill_supported: whether a step takes it (every
+// chunk of more than kMaxRows rows does; the split partials hold kMaxRows rows).
+bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim);
+void launch_attention_prefill(const float* q, const StepDev* step, int32_t n_rows, int32_t layer, int32_t n_head,
+                              int32_t n_head_kv, int32_t head_dim, float* out, hipStream_t stream);
 // Merges the splits of every (row, head) into out[row][n_head * head_dim]
 // and, when xq.q is set, quantizes the rows into xq; reads the first `slots`
 // (0: splits) split slots.

@@ -1,0 +1,79 @@
+"""Long steps: the prefill matmul tiles and the attention of whole prefill chunks."""
+import numpy as np
+import pytest
+
+import jetsonfabric_amd as jf
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [jf.Q4_K, jf.Q6_K, jf.Q2_K, jf.Q8_0]
+
+
+# Gate/up matrices of 12288 rows (192 sets of 64 rows) and 16896 rows (264): 256 rows make 384 work-groups of 128
+# tokens and 1056 of 64, the two large tile shapes. 2304 columns are nine K tiles: a chain of two and seven of one.
+@pytest.mark.parametrize("n_ff", [6144, 8448])
+@pytest.mark.parametrize("t", TYPES, ids=[jf.TYPE_NAMES[t] for t in TYPES])
+def test_long_step_matmul_equals_single_rows(t, n_ff):
+    """Rows of a long step (whole and ragged token groups) equal the same rows computed alone, bit for bit."""
+    cfg = jf.ModelConfig(n_layer=1, n_embd=2304, n_ff=n_ff, n_head=18, n_head_kv=2, n_vocab=256, n_ctx=256)
+    model = jf.Model.synthesize(cfg, type_linear=t, type_embd=t, type_output=t, seed=n_ff + t)
+    engine = jf.NativeEngine(model)
+    try:
+        for name in ("blk.0.ffn_up.weight", "blk.0.ffn_down.weight", "blk.0.attn_k.weight"):
+            cols, rows = model.tensor(name)["shape"]
+            for n_tok in (47, 241, 256):
+                x = np.random.default_rng(n_tok).standard_normal((n_tok, cols)).astype(np.float32)
+                wide = engine.matmul(name, x, rows)
+                for r in sorted({0, 15, 16, n_tok // 2, n_tok - 2, n_tok - 1}):
+                    single = engine.matmul(name, x[r:r + 1], rows)
+                    assert np.array_equal(wide[r].view(np.uint32), single[0].view(np.uint32)), f"{name} {n_tok}: row {r}"
+    finally:
+        engine.close()
+
+
+# Head dims 64 and 128, an odd query group, a few rows beyond one step, and a prompt of two chunks.
+@pytest.mark.parametrize("n_head,n_head_kv,head_dim", [(8, 2, 64), (7, 1, 128), (16, 16, 128)])
+@pytest.mark.parametrize("n", [257, 300, 2200])
+def test_chunk_attention_matches_short_steps(n_head, n_head_kv, head_dim, n):
+    """A prompt run in whole chunks reaches the logits of the same tokens run in steps of 16 rows (split-key
+    attention). Float weights: only the attention differs. Its operands are f16 hi + lo pairs (2^-21 of a value),
+    scores reach about 10, and two layers add up: 1e-4 of the largest logit is several times that."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=n_head * head_dim, n_ff=256, n_head=n_head, n_head_kv=n_head_kv,
+                         n_vocab=512, n_ctx=4096)
+    model = jf.Model.synthesize(cfg, type_linear=jf.F32, type_embd=jf.F32, type_output=jf.F32, seed=head_dim + n_head)
+    engine = jf.NativeEngine(model)
+    try:
+        tokens = [int(t) for t in np.random.default_rng(n).integers(0, cfg.n_vocab, n)]
+        s = engine.create_session(n + 16)
+        _, logits = s.prefill_greedy(tokens, logits=True)
+        ref = engine.create_session(n + 16)
+        ref.prefill_greedy(tokens[:8])
+        at = 8
+        while at < n:
+            step = tokens[at:at + 16]
+            rows = engine.step_batch([ref], [step], logits=True)[2][0]
+            at += len(step)
+        assert s.position() == ref.position() == n
+        assert np.abs(logits - rows[-1]).max() <= 1e-4 * np.abs(rows[-1]).max()
+        # the cache it leaves serves the next step
+        a = engine.step_batch([s], [[3, 5]], logits=True)[2][0]
+        b = engine.step_batch([ref], [[3, 5]], logits=True)[2][0]
+        assert np.abs(a - b).max() <= 1e-4 * np.abs(b).max()
+    finally:
+        engine.close()
+
+
+def test_step_row_limits_stay():
+    """Chunks are longer than a step may be: steps of more than 256 rows are still refused."""
+    cfg = jf.ModelConfig(n_layer=1, n_embd=512, n_ff=512, n_head=8, n_head_kv=2, n_vocab=512, n_ctx=1024)
+    engine = jf.NativeEngine(jf.Model.synthesize(cfg, type_linear=jf.Q4_K, type_embd=jf.Q4_K, type_output=jf.Q4_K, seed=1))
+    try:
+        s = engine.create_session(800)
+        s.prefill_greedy([1, 2, 3])
+        with pytest.raises(jf.JfhError, match="too many token rows"):
+            engine.step_batch([s], [[1] * 257])
+        assert s.position() == 3
+        engine.step_batch([s], [[1] * 256])
+        assert s.position() == 259
+    finally:
+        engine.close()
