@@ -2515,6 +2515,102 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32
 }
 __device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// The epilogue of a whole 64-row set: the same values as gemv_epilogue's, four rows per thread and the set's tokens
+// 256 / (threads per token) at a time, so that a thread's row arithmetic is done once, its reads (residual rows,
+// row descriptions, rotations) are all in flight together and its writes are 16 bytes wide. One element per thread
+// and turn, each turn waiting for its own read, took 10-20 us of a 48 us launch (3584 x 3584, 1024 rows).
+// vals: [token][kGemmValStride] in LDS; y_stride is a multiple of 4.
+constexpr int kGemmRows = 16 * kGemmWaves, kGemmValStride = kGemmRows + 4;
+
+#pragma clang fp contract(off)
+template <int NTOK>
+__device__ void gemm_epilogue(const GemvArgs& a, int row0, const float* vals) {
+    constexpr int NTHR = kGemmWaves * kWave, QUADS = kGemmRows / 4, TPT = NTHR / QUADS, TURNS = NTOK / TPT;
+    const int n_tok = a.n_tok;
+    if (a.mode == kSwiGLU) {
+        // output quad o4 of the set's 32: gate rows 16 (o4 / 2) + 4 (o4 % 2) .. + 3, up rows 8 further
+        constexpr int OQ = QUADS / 2, OTPT = NTHR / OQ;
+        const int o4 = threadIdx.x % OQ, tk0 = threadIdx.x / OQ, j = 16 * (o4 >> 1) + 4 * (o4 & 1);
+#pragma unroll
+        for (int u = 0; u < (NTOK + OTPT - 1) / OTPT; ++u) {
+            const int t = tk0 + u * OTPT;
+            if (t < n_tok) {
+                const f32x4 g = *reinterpret_cast<const f32x4*>(vals + t * kGemmValStride + j);
+                const f32x4 up = *reinterpret_cast<const f32x4*>(vals + t * kGemmValStride + j + kGluGroup);
+                f32x4 r;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r[k] = g[k] / (1.0F + expf(-g[k])) * up[k];
+                *reinterpret_cast<f32x4*>(a.y + static_cast<size_t>(t) * a.y_stride + row0 / 2 + 4 * o4) = r;
+            }
+        }
+        return;
+    }
+    const int j = 4 * (threadIdx.x % QUADS), tk0 = threadIdx.x / QUADS, gr = row0 + j;
+    f32x4 bias = {0.0F, 0.0F, 0.0F, 0.0F};
+    if (a.mode != kAdd && a.mat.bias) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) bias[k] = a.mat.bias[gr + k];
+    }
+    if (a.mode != kQKV) {
+        f32x4 old[TURNS];
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            const int t = min(tk0 + u * TPT, n_tok - 1);
+            old[u] = a.mode == kAdd ? *reinterpret_cast<const f32x4*>(a.y + static_cast<size_t>(t) * a.y_stride + gr) : bias;
+        }
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            const int t = tk0 + u * TPT;
+            if (t < n_tok) {
+                *reinterpret_cast<f32x4*>(a.y + static_cast<size_t>(t) * a.y_stride + gr) =
+                    *reinterpret_cast<const f32x4*>(vals + t * kGemmValStride + j) + old[u];
+            }
+        }
+        return;
+    }
+    // q | k | v: a quad is two rotated pairs of one head, or four value dims (head dims are multiples of 4)
+    const QkvOut& o = a.qkv;
+    const int hd = o.head_dim, half = hd / 2, Hq = o.n_head * hd, kv = o.n_head_kv * hd;
+    QkvRow row[TURNS];
+#pragma unroll
+    for (int u = 0; u < TURNS; ++u) row[u] = qkv_row(o, min(tk0 + u * TPT, n_tok - 1));
+    const int region = gr < Hq ? 0 : gr < Hq + kv ? 1 : 2, g = gr - (region == 0 ? 0 : region == 1 ? Hq : Hq + kv);
+    const int head = g / hd, in = g - head * hd, i = in / 2;
+    f32x4 rot[TURNS];
+    if (region < 2) {
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u)
+            rot[u] = *reinterpret_cast<const f32x4*>(o.rope + static_cast<size_t>(row[u].pos) * hd + 2 * i);
+    }
+#pragma unroll
+    for (int u = 0; u < TURNS; ++u) {
+        const int t = tk0 + u * TPT;
+        if (t >= n_tok) continue;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(vals + t * kGemmValStride + j) + bias;
+        const size_t cache_head = static_cast<size_t>(o.layer) * o.n_head_kv + head;
+        if (region == 2) {
+            // 16-position tiles, transposed within a tile, as qkv_store
+            global_ptr<uint16_t> vc = as_global(row[u].v);
+            const size_t at = (cache_head * row[u].capacity + (row[u].pos & ~15)) * hd + static_cast<size_t>(in) * 16 + (row[u].pos & 15);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) vc[at + 16 * k] = f2h(v[k]);
+            continue;
+        }
+        const float a0 = v[0] * rot[u][0] - v[1] * rot[u][1], b0 = v[0] * rot[u][1] + v[1] * rot[u][0];
+        const float a1 = v[2] * rot[u][2] - v[3] * rot[u][3], b1 = v[2] * rot[u][3] + v[3] * rot[u][2];
+        if (region == 0) {
+            float* q = o.q + static_cast<size_t>(t) * Hq + head * hd + i;
+            *reinterpret_cast<float2*>(q) = make_float2(a0, a1);
+            *reinterpret_cast<float2*>(q + half) = make_float2(b0, b1);
+        } else {
+            global_ptr<uint16_t> kc = as_global(row[u].k) + (cache_head * row[u].capacity + row[u].pos) * hd + i;
+            *(global_ptr<uint32_t>) kc = f2h(a0) | (static_cast<uint32_t>(f2h(a1)) << 16);
+            *(global_ptr<uint32_t>) (kc + half) = f2h(b0) | (static_cast<uint32_t>(f2h(b1)) << 16);
+        }
+    }
+}
+#pragma clang fp contract(on)
+
 template <uint32_t TYPE, int TP, int OCC>
 __global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a, int32_t n_rg) {
     constexpr int NW = kGemmWaves, NTHR = NW * kWave, NTOK = 16 * TP, NROW = 16 * NW;
@@ -2522,7 +2618,7 @@ __global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a,
     constexpr uint32_t TB = tile_bytes(TYPE);
     constexpr int CPW = NTOK / (4 * NW);  // 1 KB copies (four token rows) per wave of a staged tile
     static_assert(NTOK % (4 * NW) == 0 && 2 * NTOK <= NTHR, "whole copies per wave, half a token's sums per thread");
-    constexpr int VSTRIDE = NROW + 1;  // epilogue row stride (floats)
+    constexpr int VSTRIDE = kGemmValStride;  // epilogue row stride (floats)
     constexpr int CODES = 2 * NTOK * 256, VALS = NTOK * VSTRIDE * 4;
     constexpr int SIDE = Q8 ? 8 : 1;  // scales per token and tile
     __shared__ __align__(16) uint8_t codes[CODES > VALS ? CODES : VALS];  // then the epilogue's values
@@ -2733,16 +2829,17 @@ __global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a,
     float* vals = reinterpret_cast<float*>(&codes[0]);
 #pragma unroll
     for (int tl = 0; tl < TP; ++tl) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vals[(16 * tl + i) * VSTRIDE + 16 * wave + 4 * G + j] = total[tl][j];
+        *reinterpret_cast<f32x4*>(vals + (16 * tl + i) * VSTRIDE + 16 * wave + 4 * G) =
+            f32x4{total[tl][0], total[tl][1], total[tl][2], total[tl][3]};
     }
     __syncthreads();
     const int row0 = set * NROW, nrows = min(NROW, static_cast<int>(a.mat.rows) - row0);
     const GemvArgs out = token_slice(a, t0, nt);
-    auto value = [&](int j, int tk) { return vals[tk * VSTRIDE + j]; };
-    // whole sets divide by a constant
-    if (nrows == NROW) gemv_epilogue<NTHR, kNoLogits>(out, row0, NROW, value, nullptr);
-    else gemv_epilogue<NTHR, kNoLogits>(out, row0, nrows, value, nullptr);
+    if (nrows == NROW && (a.mode == kQKV || a.y_stride % 4 == 0)) {
+        gemm_epilogue<NTOK>(out, row0, vals);
+    } else {
+        gemv_epilogue<NTHR, kNoLogits>(out, row0, nrows, [&](int j, int tk) { return vals[tk * VSTRIDE + j]; }, nullptr);
+    }
 }
 
 // The folded tiles for steps whose grid is too small for the long-step matmul: the decode matmul's eight waves (wave
