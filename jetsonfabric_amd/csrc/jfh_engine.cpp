@@ -46,26 +46,93 @@ bool quantized(uint32_t type) { return type == kQ4_K || type == kQ6_K || type ==
 // The last prefill's metrics per calling thread (Engine::last_prefill_metrics).
 thread_local PrefillMetrics t_last_prefill;
 
+// ------------------------------------------------------------------ cache buffers
+void* CachePool::take(size_t bytes, size_t& size) {
+    constexpr size_t kUnit = size_t{1} << 20;
+    const size_t want = (bytes + kUnit - 1) / kUnit * kUnit;
+    {
+        // the smallest kept buffer that fits and wastes no more than a quarter
+        std::lock_guard lock(mutex_);
+        size_t best = free_.size();
+        for (size_t i = 0; i < free_.size(); ++i) {
+            if (free_[i].size < want || free_[i].size > want + want / 4) continue;
+            if (best == free_.size() || free_[i].size < free_[best].size) best = i;
+        }
+        if (best < free_.size()) {
+            const Buffer b = free_[best];
+            free_.erase(free_.begin() + static_cast<std::ptrdiff_t>(best));
+            held_ -= b.size;
+            size = b.size;
+            return b.p;
+        }
+    }
+    void* p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void) hipGetLastError();
+        drain();
+        if (hipMalloc(&p, want) != hipSuccess) return nullptr;
+    }
+    size = want;
+    return p;
+}
+
+void CachePool::put(void* p, size_t size) {
+    if (p == nullptr) return;
+    std::vector<Buffer> out;
+    {
+        std::lock_guard lock(mutex_);
+        if (closed_ || size > kBytes) {
+            out.push_back({p, size});
+        } else {
+            free_.push_back({p, size});
+            held_ += size;
+            while (free_.size() > kBuffers || held_ > kBytes) {  // the longest kept ones go first
+                held_ -= free_.front().size;
+                out.push_back(free_.front());
+                free_.erase(free_.begin());
+            }
+        }
+    }
+    for (const Buffer& b : out) (void) hipFree(b.p);
+}
+
+void CachePool::drain() {
+    std::vector<Buffer> out;
+    {
+        std::lock_guard lock(mutex_);
+        out.swap(free_);
+        held_ = 0;
+    }
+    for (const Buffer& b : out) (void) hipFree(b.p);
+}
+
+void CachePool::close() {
+    {
+        std::lock_guard lock(mutex_);
+        closed_ = true;
+    }
+    drain();
+}
+
 // ------------------------------------------------------------------ Session
 Session::Session(Engine* engine, uint32_t capacity)
     : engine_(engine), capacity_(capacity), stride_((std::max<uint32_t>(capacity, 16) + 15) / 16 * 16) {
     const ModelParams& p = engine->params();
     const size_t elems = static_cast<size_t>(engine->resident_layers()) * p.n_head_kv * stride_ * p.head_dim;
     kv_bytes_ = 2 * elems * sizeof(uint16_t);
-    hip_check(hipMalloc(&k_, elems * sizeof(uint16_t)), "allocate K cache");
-    if (hipMalloc(&v_, elems * sizeof(uint16_t)) != hipSuccess) {
-        (void) hipFree(k_);
-        fail(Status::OutOfMemory, "allocate V cache");
+    pool_ = engine->pool_;
+    k_ = static_cast<uint16_t*>(pool_->take(kv_bytes_, buffer_bytes_));
+    if (k_ == nullptr) fail(Status::OutOfMemory, "allocate K and V cache");
+    v_ = k_ + elems;
+    // every use of the cache is ordered behind this on the engine's stream
+    const hipError_t e = hipMemsetAsync(k_, 0, kv_bytes_, engine->stream());
+    if (e != hipSuccess) {
+        pool_->put(k_, buffer_bytes_);
+        hip_check(e, "clear KV cache");
     }
-    hip_check(hipMemsetAsync(k_, 0, elems * sizeof(uint16_t), engine->stream()), "clear K cache");
-    hip_check(hipMemsetAsync(v_, 0, elems * sizeof(uint16_t), engine->stream()), "clear V cache");
-    hip_check(hipStreamSynchronize(engine->stream()), "clear KV cache");
 }
 
-Session::~Session() {
-    (void) hipFree(k_);
-    (void) hipFree(v_);
-}
+Session::~Session() { pool_->put(k_, buffer_bytes_); }
 
 void Session::rollback(uint32_t n) {
     // qwen2_architecture.cpp:818-823: only the decoded suffix can be removed;
@@ -468,6 +535,7 @@ Engine::Engine(const HostModel& model, const EngineOptions& options) : params_(m
 }
 
 Engine::~Engine() {
+    pool_->close();
     for (auto& [key, exec] : graphs_) (void) hipGraphExecDestroy(exec);
     for (void* p : allocations_) (void) hipFree(p);
     if (partial_) (void) hipFree(partial_);
@@ -497,7 +565,10 @@ void Engine::ensure_capacity(uint32_t capacity) {
                                                                 static_cast<int32_t>(p.head_dim), splits_);
     if (partial_) (void) hipFree(partial_);
     partial_ = nullptr;
-    hip_check(hipMalloc(&partial_, partial_floats * sizeof(float)), "allocate attention partials");
+    if (hipMalloc(&partial_, partial_floats * sizeof(float)) != hipSuccess) {
+        pool_->drain();
+        hip_check(hipMalloc(&partial_, partial_floats * sizeof(float)), "allocate attention partials");
+    }
     capacity_max_ = cap;
     for (auto& [key, exec] : graphs_) (void) hipGraphExecDestroy(exec);
     graphs_.clear();

@@ -58,6 +58,32 @@ struct BufferMetrics {
     uint64_t prefill_host_input_bytes = 0;
 };
 
+// Cache buffers of closed sessions, kept for the next ones: allocating and freeing device memory took longer than a
+// short prompt's first layers (7B, 100 rows: about 150 of 980 us per request). At most kBytes in kBuffers buffers,
+// given back with the engine and whenever an allocation fails. Sessions share it, since one may outlive its engine
+// and may be closed on any thread. Every step has finished when it returns, so a closed session's buffer is idle.
+class CachePool {
+public:
+    static constexpr size_t kBytes = size_t{256} << 20;
+    static constexpr size_t kBuffers = 8;
+    ~CachePool() { close(); }
+    // A buffer of at least `bytes` (its size is stored in `size`), nullptr when the device has no memory left.
+    void* take(size_t bytes, size_t& size);
+    void put(void* p, size_t size);
+    void drain();
+    void close();  // drains; buffers put back later are freed
+
+private:
+    struct Buffer {
+        void* p;
+        size_t size;
+    };
+    std::mutex mutex_;
+    std::vector<Buffer> free_;
+    size_t held_ = 0;
+    bool closed_ = false;
+};
+
 class Session {
 public:
     ~Session();
@@ -81,6 +107,8 @@ private:
     uint32_t stride_;  // allocated positions per (layer, kv head): capacity rounded up to 16
     uint32_t position_ = 0;
     uint32_t prefill_position_ = 0;
+    std::shared_ptr<CachePool> pool_;
+    size_t buffer_bytes_ = 0;  // of the buffer that holds K, then V
     uint16_t* k_ = nullptr;  // [resident layer][kv head][stride][head_dim]
     uint16_t* v_ = nullptr;  // [resident layer][kv head][stride / 16][head_dim][16] (16-position tiles)
     uint64_t kv_bytes_ = 0;
@@ -247,6 +275,7 @@ private:
     hipEvent_t ev_order_ = nullptr;  // orders the allocation-free matmul after the caller's stream
     double attn_kv_bytes_ = 0.0;  // K/V bytes one layer's attention reads in the step being recorded
     void* device_alloc(size_t bytes);
+    std::shared_ptr<CachePool> pool_ = std::make_shared<CachePool>();
 
     ModelParams params_;
     EngineOptions options_;

@@ -77,3 +77,27 @@ def test_step_row_limits_stay():
         assert s.position() == 259
     finally:
         engine.close()
+
+
+def test_reused_cache_buffers_start_clean():
+    """Sessions opened after others were closed (their buffers are kept, more of them than the engine keeps) give the
+    logits of a fresh engine, also with another capacity; a session may be closed after its engine."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=512, n_ff=512, n_head=8, n_head_kv=2, n_vocab=512, n_ctx=2048)
+    model = jf.Model.synthesize(cfg, type_linear=jf.Q4_K, type_embd=jf.Q4_K, type_output=jf.Q4_K, seed=9)
+    fresh, used = jf.NativeEngine(model), jf.NativeEngine(model)
+    tokens = [int(t) for t in np.random.default_rng(2).integers(0, cfg.n_vocab, 40)]
+    many = [used.create_session(c) for c in (64, 64, 100, 1500, 1500, 700, 64, 64, 64, 300, 2000, 64)]
+    for s in many:
+        s.prefill_greedy(tokens[::-1])
+    for s in many:
+        s.close()
+    for capacity in (64, 60, 1500, 2000, 90):
+        a, b = fresh.create_session(capacity), used.create_session(capacity)
+        la, lb = a.prefill_greedy(tokens, logits=True)[1], b.prefill_greedy(tokens, logits=True)[1]
+        assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)), capacity
+        a.close()
+        b.close()
+    late = used.create_session(64)
+    used.close()
+    late.close()
+    fresh.close()
