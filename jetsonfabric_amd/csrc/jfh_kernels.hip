@@ -2847,18 +2847,17 @@ __global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a,
 // K tile's activations (lane (i, G): token i's bytes 64 G .. 64 G + 63, its code sums and scales) once and runs them
 // against the R row groups' folded weight operands, the next weight tile in flight while one runs; no LDS and no
 // barrier until the waves' partials are summed in wave order, so every row equals the decode row bit for bit.
-template <uint32_t TYPE, int R>
+template <uint32_t TYPE, int R, int TP>
 __global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg) {
     constexpr int W = kMmWaves;
-    constexpr bool Q8 = TYPE == 7;
     constexpr uint32_t TB = tile_bytes(TYPE);
     using T = GemmTile<TYPE>;
-    __shared__ float red[W][16][16 * R];  // [wave][token][row]
-    __shared__ float vals[16][16 * R];
-    const int n_tok = a.n_tok, n_tt = (n_tok + 15) / 16;
-    // work-group k runs on XCD k % 8: the token tiles of one row-group set share an XCD (and its L2)
+    __shared__ float red[W][16 * TP][16 * R];  // [wave][token][row]
+    __shared__ float vals[16 * TP][16 * R];
+    const int n_tok = a.n_tok, n_grp = ((n_tok + 15) / 16 + TP - 1) / TP;
+    // work-group k runs on XCD k % 8: the token groups of one row-group set share an XCD (and its L2)
     const int q = static_cast<int>(blockIdx.x) >> 3;
-    const int tt = q % n_tt, set = (q / n_tt) * 8 + static_cast<int>(blockIdx.x & 7u);
+    const int grp = q % n_grp, set = (q / n_grp) * 8 + static_cast<int>(blockIdx.x & 7u);
     const int rg0 = set * R;
     if (rg0 >= n_rg) return;
     const int nrg = min(R, n_rg - rg0);
@@ -2866,43 +2865,39 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
     const int i = lane & 15, G = lane >> 4;
-    const int t0 = 16 * tt, nt = min(16, n_tok - t0);
+    const int t0 = 16 * TP * grp, nt = min(16 * TP, n_tok - t0);
     const GemvArgs out = token_slice(a, t0, nt);
     const Act8 xq = a.xq;
-    // the lane's token (rows past the step repeat its last row; never stored)
-    const uint32_t tok = static_cast<uint32_t>(min(t0 + i, n_tok - 1));
+    // the lane's tokens (rows past the step repeat its last row; never stored)
+    uint32_t tok[TP];
+#pragma unroll
+    for (int tl = 0; tl < TP; ++tl) tok[tl] = static_cast<uint32_t>(min(t0 + 16 * tl + i, n_tok - 1));
     const uint8_t* base = a.mat.data + static_cast<size_t>(rg0) * nb * TB;
     auto load_raw = [&](int rr, int b) { return T::load(base + (static_cast<size_t>(rr) * nb + b) * TB, lane); };
-    float acc[R][4];
+    float acc[R][TP][4];
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[rr][j] = 0.0F;
+        for (int tl = 0; tl < TP; ++tl) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[rr][tl][j] = 0.0F;
+        }
     }
     typename T::Raw cur = load_raw(0, min(wave, nb - 1));
     for (int b = wave; b < nb; b += W) {
-        const uint4* src = reinterpret_cast<const uint4*>(xq.q + (tok * static_cast<uint32_t>(K) + 256u * b + 64u * G));
-        uint4 xa[4];
+        u32x4 xa[TP][4];
+        f16x4 xs[TP];
+        float xd[TP];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) xa[m] = src[m];
-        f16x4 xs = {};
-        float xd[Q8 ? 8 : 1];
-        long av[8];
-        if constexpr (Q8) {
-            const f32x4* ds = reinterpret_cast<const f32x4*>(xq.d + (tok * static_cast<uint32_t>(K / 32) + 8u * b));
-            const f32x4 d0 = ds[0], d1 = ds[1];
+        for (int tl = 0; tl < TP; ++tl) {
+            const u32x4* src = reinterpret_cast<const u32x4*>(xq.q + (tok[tl] * static_cast<uint32_t>(K) + 256u * b + 64u * G));
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                xd[k] = d0[k];
-                xd[4 + k] = d1[k];
-            }
-            wide_a_operands(xa, av);
-        } else {
-            xd[0] = xq.d[tok * static_cast<uint32_t>(nb) + b];
+            for (int m = 0; m < 4; ++m) xa[tl][m] = src[m];
+            xd[tl] = xq.d[tok[tl] * static_cast<uint32_t>(nb) + b];
             if constexpr (T::kMins) {
-                const uint2 sw = *reinterpret_cast<const uint2*>(xq.s + (tok * static_cast<uint32_t>(K / 16) + 16u * b + 4u * G));
-                xs = f16x4{static_cast<_Float16>(static_cast<int16_t>(sw.x & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.x >> 16)),
-                           static_cast<_Float16>(static_cast<int16_t>(sw.y & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.y >> 16))};
+                const uint2 sw = *reinterpret_cast<const uint2*>(xq.s + (tok[tl] * static_cast<uint32_t>(K / 16) + 16u * b + 4u * G));
+                xs[tl] = f16x4{static_cast<_Float16>(static_cast<int16_t>(sw.x & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.x >> 16)),
+                               static_cast<_Float16>(static_cast<int16_t>(sw.y & 0xFFFFu)), static_cast<_Float16>(static_cast<int16_t>(sw.y >> 16))};
             }
         }
 #pragma unroll
@@ -2910,16 +2905,11 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg
             // the next weight tile (the next row group's, else the wave's next K tile's first; clamped)
             const typename T::Raw nxt = rr + 1 < nrg ? load_raw(rr + 1, b) : load_raw(0, min(b + W, nb - 1));
             if (rr < nrg) {
-                if constexpr (Q8) {
-                    i32x4 A[8];
+                u32x4 B[T::kChains][4];
+                typename T::Scale sc;
+                T::fold(cur, lane, B, sc);
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) A[k] = mfma_i8(pack2(cur.w[k].x, cur.w[k].y), av[k]);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[rr][j] += T::tile_term(cur, j, A, xd);
-                } else {
-                    u32x4 B[T::kChains][4];
-                    typename T::Scale sc;
-                    T::fold(cur, lane, B, sc);
+                for (int tl = 0; tl < TP; ++tl) {
                     i32x4 D[T::kChains];
 #pragma unroll
                     for (int c = 0; c < T::kChains; ++c) D[c] = i32x4{0, 0, 0, 0};
@@ -2928,16 +2918,16 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg
 #pragma unroll
                         for (int c = 0; c < T::kChains; ++c) {
                             D[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, B[c][m]),
-                                                                         __builtin_bit_cast(i32x4, xa[m]), D[c], 0, 0, 0);
+                                                                         __builtin_bit_cast(i32x4, xa[tl][m]), D[c], 0, 0, 0);
                         }
                     }
                     f32x4 ms = {0.0F, 0.0F, 0.0F, 0.0F};
-                    if constexpr (T::kMins) ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sc.mins, xs, ms, 0, 0, 0);
+                    if constexpr (T::kMins) ms = __builtin_amdgcn_mfma_f32_16x16x16f16(sc.mins, xs[tl], ms, 0, 0, 0);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         int isum = D[0][j];
                         if constexpr (T::kChains == 2) isum += static_cast<int>(static_cast<uint32_t>(D[1][j]) << T::kShift);
-                        acc[rr][j] = T::step(acc[rr][j], xd[0], sc, j, isum, ms[j]);
+                        acc[rr][tl][j] = T::step(acc[rr][tl][j], xd[tl], sc, j, isum, ms[j]);
                     }
                 }
             }
@@ -2948,10 +2938,13 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_fold(GemvArgs a, int32_t n_rg
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) red[wave][i][16 * rr + 4 * G + j] = acc[rr][j];
+        for (int tl = 0; tl < TP; ++tl) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[wave][16 * tl + i][16 * rr + 4 * G + j] = acc[rr][tl][j];
+        }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * 16 * nrg; e += kMmThreads) {
+    for (int e = threadIdx.x; e < 16 * TP * 16 * nrg; e += kMmThreads) {
         const int tk = e / (16 * nrg), r = e - tk * 16 * nrg;
         float v = 0.0F;
 #pragma unroll
@@ -4174,26 +4167,17 @@ constexpr int kWideQ4kMinWgs = 256;
 
 bool wide_matmul_supported(uint32_t type) { return type == 7 || type == 9 || type == 11 || type == 13; }
 
-// Measured on 7B-shaped layers: Q4_K and Q8_0 from 9 rows; Q6_K and Q2_K,
-// whose 16-value sub-blocks take two half-masked MFMAs per 32 values, only
-// beyond one 16-slot token-quad group.
+// From 9 rows the wide kernels outrun the token quads for every format (9 rows: 3584 x 18944 Q6_K 29 us in quads, 19
+// here; 5120 x 27648 Q2_K 39 and 20; 2048 x 1536 Q6_K 5.4 and 4.2).
 constexpr int32_t kWideFromRows = 9;
-int32_t wide_min_rows(uint32_t type) {
-    switch (type) {
-    case 7:
-    case 11: return kWideFromRows;
-    case 9:
-    case 13: return kQuadGroupRows + 1;
-    default: return 0;
-    }
-}
+int32_t wide_min_rows(uint32_t type) { return wide_matmul_supported(type) ? kWideFromRows : 0; }
 
 // Which kernel a layer matrix's step takes, by the work-groups that 64 rows x 16 TP tokens make of it (256 CUs;
 // measured over 9..2048 rows on matrices of 1536..55296 rows). Each K tile costs a wave of the long-step matmul about
 // 1 us of latency however few tokens it carries, so below about 1.5 work-groups per CU the K-split kernel is faster
 // (7B Q4_K down, 56 row sets: 160 rows 79 us against 83, 256 rows 109 against 86), unless K is so short that its
 // eight waves have no two tiles each (2048 x 1536 Q6_K, 256 rows: 12.7 against 10.4).
-constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192;
+constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192, kGemmQ8OneWgs = 480;
 constexpr int kGemmFillWgs = 1024;  // four waves per SIMD everywhere
 constexpr int kGemmShortTiles = 8;
 
@@ -4203,9 +4187,9 @@ void gemm(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
     launch(k_mm_gemm<TYPE, TP, OCC>, dim3((wgs + 7) / 8 * 8), dim3(kGemmWaves * kWave), 0, stream, a, n_rg);
 }
 
-template <uint32_t TYPE, int R>
+template <uint32_t TYPE, int R, int TP>
 void fold(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
-    launch(k_mm_fold<TYPE, R>, dim3(((n_rg + R - 1) / R + 7) / 8 * 8 * n_tt), dim3(kMmThreads), 0, stream, a, n_rg);
+    launch(k_mm_fold<TYPE, R, TP>, dim3(((n_rg + R - 1) / R + 7) / 8 * 8 * ((n_tt + TP - 1) / TP)), dim3(kMmThreads), 0, stream, a, n_rg);
 }
 
 // A K-quant layer matrix.
@@ -4229,8 +4213,8 @@ void folded(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
     else if (n_tt >= 3 && wgs(4) >= kGemmMinWgs) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
     else if (n_tt >= 2 && wgs(2) >= (short_k ? kGemmShortWgs : kGemmMinWgs)) gemm<TYPE, 2, 3>(a, n_rg, n_tt, stream);
     // one row group per work-group only while that is at most a work-group per CU
-    else if (n_rg * n_tt <= 256) fold<TYPE, 1>(a, n_rg, n_tt, stream);
-    else fold<TYPE, 2>(a, n_rg, n_tt, stream);
+    else if (n_rg * n_tt <= 256) fold<TYPE, 1, 1>(a, n_rg, n_tt, stream);
+    else fold<TYPE, 2, 1>(a, n_rg, n_tt, stream);
     check(hipGetLastError(), "wide matmul launch");
 }
 
@@ -4254,10 +4238,14 @@ void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
         return;
     }
     if (!merged && n_tt >= 2) {
-        // Q8_0, bound by its float step per 32-value block: one tile shape
-        const int wgs = (n_rg + kGemmWaves - 1) / kGemmWaves * ((n_tt + 1) / 2);
-        if (wgs >= (static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs)) {
-            gemm<7, 2, 3>(a, n_rg, n_tt, stream);
+        // Q8_0, bound by its float step per 32-value block: two token tiles, or one while that makes about two
+        // work-groups per CU (1536 x 8960, 333 rows, 504 work-groups: 55 us on the K-split kernel, 47 here; 256 rows,
+        // 384: 39 and 45)
+        const int n_sets = (n_rg + kGemmWaves - 1) / kGemmWaves, wgs = n_sets * ((n_tt + 1) / 2);
+        const bool two = wgs >= (static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs);
+        if (two || n_sets * n_tt >= kGemmQ8OneWgs) {
+            if (two) gemm<7, 2, 3>(a, n_rg, n_tt, stream);
+            else gemm<7, 1, 4>(a, n_rg, n_tt, stream);
             check(hipGetLastError(), "wide matmul launch");
             return;
         }
