@@ -2843,7 +2843,7 @@ __global__ __launch_bounds__(kGemmWaves * kWave, OCC) void k_mm_gemm(GemvArgs a,
 }
 
 // The folded tiles for steps whose grid is too small for the long-step matmul: the decode matmul's eight waves (wave
-// w takes the K tiles w, w + 8, ...), R consecutive row groups and one 16-token tile per work-group. A wave loads its
+// w takes the K tiles w, w + 8, ...), R consecutive row groups and TP 16-token tiles per work-group. A wave loads its
 // K tile's activations (lane (i, G): token i's bytes 64 G .. 64 G + 63, its code sums and scales) once and runs them
 // against the R row groups' folded weight operands, the next weight tile in flight while one runs; no LDS and no
 // barrier until the waves' partials are summed in wave order, so every row equals the decode row bit for bit.
@@ -4214,7 +4214,17 @@ void folded(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
     else if (n_tt >= 2 && wgs(2) >= (short_k ? kGemmShortWgs : kGemmMinWgs)) gemm<TYPE, 2, 3>(a, n_rg, n_tt, stream);
     // one row group per work-group only while that is at most a work-group per CU
     else if (n_rg * n_tt <= 256) fold<TYPE, 1, 1>(a, n_rg, n_tt, stream);
-    else fold<TYPE, 2, 1>(a, n_rg, n_tt, stream);
+    else {
+        // Two row groups x one or two token tiles per work-group. Two fold a weight tile half as often but leave half
+        // the work-groups, which pays where one tile needs a second work-group on some CUs and two do not (5120 x
+        // 13824 Q4_K, 18 rows: 320 work-groups 27 us, 160 21 us; 33 rows: 480 27 us, 320 43 us), where two fit one
+        // resident round of two per CU and one does not (3584 x 18944, 100 rows: 784 60 us, 448 54 us), and always for
+        // Q6_K, whose fold is the longest (3584 x 18944, 200 rows: 116 and 100 us).
+        const int one = (n_rg + 1) / 2 * n_tt, two = (n_rg + 1) / 2 * ((n_tt + 1) / 2);
+        const bool tiles2 = one > 256 && (TYPE == 13 || two <= 256 || (one > 512 && two > 384 && two <= 512));
+        if (tiles2) fold<TYPE, 2, 2>(a, n_rg, n_tt, stream);
+        else fold<TYPE, 2, 1>(a, n_rg, n_tt, stream);
+    }
     check(hipGetLastError(), "wide matmul launch");
 }
 
