@@ -428,7 +428,7 @@ typedef struct jfh_generation_stats {
     double decode_tokens_per_second;      /* tokens after the first / decode_ms */
     double end_to_end_tokens_per_second;  /* sampled tokens / (time to first token + decode_ms) */
     /* PrefillMetrics (native_inference.hpp:71-78): the prompt's steps */
-    uint32_t prefill_plan_reused;         /* every prefill step shape's captured graph existed already */
+    uint32_t prefill_plan_reused;         /* no step graph had to be captured (chunks beyond a step run without one) */
     uint32_t prefill_attention_matrix_cores; /* attention on MFMA (head dim 64 or 128) */
     double prefill_planning_ms;           /* capturing and instantiating new step graphs */
     double prefill_allocation_ms;         /* the session's KV cache allocation and clearing */
