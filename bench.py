@@ -326,7 +326,8 @@ def main() -> int:
     log("verify profile (ms/step): " + ", ".join(f"{p['kernel']} {p['ms']:.3f}" for p in vprof[:8]))
     session.close()
     # one prefill chunk at the position of the prompt's last chunk, in a session no larger than the one above
-    n_chunk = min(engine.prefill_chunk, context)
+    # (the second half of a prompt that fits one chunk: a profiled session has been prefilled)
+    n_chunk = min(engine.prefill_chunk, (context + 1) // 2)
     psess = engine.create_session(context + 8)
     if context > n_chunk:
         psess.prefill_greedy(prompt[:context - n_chunk])
