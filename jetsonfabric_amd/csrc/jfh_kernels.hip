@@ -4173,13 +4173,57 @@ constexpr int32_t kWideFromRows = 9;
 int32_t wide_min_rows(uint32_t type) { return wide_matmul_supported(type) ? kWideFromRows : 0; }
 
 // Which kernel a layer matrix's step takes, by the work-groups that 64 rows x 16 TP tokens make of it (256 CUs;
-// measured over 9..2048 rows on matrices of 1536..55296 rows). Each K tile costs a wave of the long-step matmul about
+// measured over 9..2048 rows on matrices of 512..55296 rows). Each K tile costs a wave of the long-step matmul about
 // 1 us of latency however few tokens it carries, so below about 1.5 work-groups per CU the K-split kernel is faster
 // (7B Q4_K down, 56 row sets: 160 rows 79 us against 83, 256 rows 109 against 86), unless K is so short that its
 // eight waves have no two tiles each (2048 x 1536 Q6_K, 256 rows: 12.7 against 10.4).
+constexpr int kCus = 256;
 constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192, kGemmQ8OneWgs = 480;
 constexpr int kGemmFillWgs = 1024;  // four waves per SIMD everywhere
 constexpr int kGemmShortTiles = 8;
+
+namespace {
+
+MmRoute fold_route(uint32_t type, int n_rg, int n_tt) {
+    // one row group per work-group only while that is at most a work-group per CU
+    if (n_rg * n_tt <= kCus) return {MmKernel::kFold, 1, 1};
+    // Two row groups x one or two token tiles per work-group. The time goes with the work-groups that the busiest CU
+    // runs, and a work-group of two token tiles takes 1.8 times one of one tile (median over 23 matrices, 33..256
+    // rows: Q4_K 1.80, Q2_K 1.70), for Q6_K, whose fold is the longest, 1.4 times (1.45). Q4_K: 5120 x 13824, 18 rows,
+    // 2 work-groups of one tile per CU 27 us, 1 of two 21; 3584 x 18944, 100 rows, 4 and 2: 60 and 54; 7168 x 5120,
+    // 33 rows, 3 and 2: 15.7 and 21.1.
+    const int pairs = (n_rg + 1) / 2;
+    const int one = (pairs * n_tt + kCus - 1) / kCus, two = (pairs * ((n_tt + 1) / 2) + kCus - 1) / kCus;
+    const int tenths = type == 13 ? 14 : 18;
+    return {MmKernel::kFold, 2, n_tt > 1 && tenths * two < 10 * one ? 2 : 1};
+}
+
+}  // namespace
+
+MmRoute mm_route(uint32_t type, uint32_t rows, uint32_t cols, int32_t n_tok) {
+    const int n_rg = (static_cast<int>(rows) + 15) / 16, n_tt = (n_tok + 15) / 16;
+    const int n_sets = (n_rg + kGemmWaves - 1) / kGemmWaves;
+    auto wgs = [&](int tp) { return n_sets * ((n_tt + tp - 1) / tp); };
+    const int two_wgs = static_cast<int>(cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs;
+    if (type == 7) {
+        // Q8_0, bound by its float step per 32-value block: two token tiles, or one while that makes about two
+        // work-groups per CU (1536 x 8960, 333 rows, 504 work-groups: 55 us on the K-split kernel, 47 here; 256 rows,
+        // 384: 39 and 45)
+        if (n_tt >= 2 && wgs(2) >= two_wgs) return {MmKernel::kGemm, kGemmWaves, 2};
+        if (n_tt >= 2 && wgs(1) >= kGemmQ8OneWgs) return {MmKernel::kGemm, kGemmWaves, 1};
+        // as many token tiles per work-group as still leave kWideMinWgs work-groups
+        int tiles = std::min(n_tt, kWideTpw);
+        while (tiles > 1 && n_rg * ((n_tt + tiles - 1) / tiles) < kWideMinWgs) --tiles;
+        return {MmKernel::kWide, 1, tiles};
+    }
+    // one or two token tiles against many row groups stream the weights from HBM
+    if (type == 11 && n_tt <= 2 && n_sets >= kWideQ4kMinWgs) return {MmKernel::kStream, kWideQ4kWaves, n_tt};
+    if (n_tt >= 3 && wgs(4) >= kGemmFillWgs) return {MmKernel::kGemm, kGemmWaves, 4};
+    if (n_tt >= 16 && wgs(8) >= kGemmMinWgs) return {MmKernel::kGemm, kGemmWaves, 8};
+    if (n_tt >= 3 && wgs(4) >= kGemmMinWgs) return {MmKernel::kGemm, kGemmWaves, 4};
+    if (n_tt >= 2 && wgs(2) >= two_wgs) return {MmKernel::kGemm, kGemmWaves, 2};
+    return fold_route(type, n_rg, n_tt);
+}
 
 template <uint32_t TYPE, int TP, int OCC>
 void gemm(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
@@ -4194,38 +4238,16 @@ void fold(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
 
 // A K-quant layer matrix.
 template <uint32_t TYPE>
-void folded(const GemvArgs& a, int n_rg, int n_tt, hipStream_t stream) {
-    const int n_sets = (n_rg + kGemmWaves - 1) / kGemmWaves;
-    auto wgs = [&](int tp) { return n_sets * ((n_tt + tp - 1) / tp); };
-    const bool short_k = static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles;
-    if constexpr (TYPE == 11) {
-        // one or two token tiles against many row groups stream the weights from HBM
-        if (n_tt <= 2 && n_sets >= kWideQ4kMinWgs) {
-            const dim3 g((n_sets + 7) / 8 * 8), b(kWideQ4kWaves * kWave);
-            if (n_tt == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg, 2);
-            else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg, 1);
-            check(hipGetLastError(), "wide matmul launch");
-            return;
-        }
-    }
-    if (n_tt >= 3 && wgs(4) >= kGemmFillWgs) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
-    else if (n_tt >= 16 && wgs(8) >= kGemmMinWgs) gemm<TYPE, 8, 2>(a, n_rg, n_tt, stream);
-    else if (n_tt >= 3 && wgs(4) >= kGemmMinWgs) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
-    else if (n_tt >= 2 && wgs(2) >= (short_k ? kGemmShortWgs : kGemmMinWgs)) gemm<TYPE, 2, 3>(a, n_rg, n_tt, stream);
-    // one row group per work-group only while that is at most a work-group per CU
-    else if (n_rg * n_tt <= 256) fold<TYPE, 1, 1>(a, n_rg, n_tt, stream);
-    else {
-        // Two row groups x one or two token tiles per work-group. Two fold a weight tile half as often but leave half
-        // the work-groups, which pays where one tile needs a second work-group on some CUs and two do not (5120 x
-        // 13824 Q4_K, 18 rows: 320 work-groups 27 us, 160 21 us; 33 rows: 480 27 us, 320 43 us), where two fit one
-        // resident round of two per CU and one does not (3584 x 18944, 100 rows: 784 60 us, 448 54 us), and always for
-        // Q6_K, whose fold is the longest (3584 x 18944, 200 rows: 116 and 100 us).
-        const int one = (n_rg + 1) / 2 * n_tt, two = (n_rg + 1) / 2 * ((n_tt + 1) / 2);
-        const bool tiles2 = one > 256 && (TYPE == 13 || two <= 256 || (one > 512 && two > 384 && two <= 512));
-        if (tiles2) fold<TYPE, 2, 2>(a, n_rg, n_tt, stream);
+void folded(const GemvArgs& a, const MmRoute& r, int n_rg, int n_tt, hipStream_t stream) {
+    if (r.kernel == MmKernel::kGemm) {
+        if (r.tiles == 8) gemm<TYPE, 8, 2>(a, n_rg, n_tt, stream);
+        else if (r.tiles == 4) gemm<TYPE, 4, 4>(a, n_rg, n_tt, stream);
+        else gemm<TYPE, 2, 3>(a, n_rg, n_tt, stream);
+    } else {
+        if (r.groups == 1) fold<TYPE, 1, 1>(a, n_rg, n_tt, stream);
+        else if (r.tiles == 2) fold<TYPE, 2, 2>(a, n_rg, n_tt, stream);
         else fold<TYPE, 2, 1>(a, n_rg, n_tt, stream);
     }
-    check(hipGetLastError(), "wide matmul launch");
 }
 
 void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
@@ -4241,28 +4263,27 @@ void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
     const GemvArgs& a = a_in;
     const int n_rg = (static_cast<int>(a.mat.rows) + 15) / 16, n_tt = (a.n_tok + 15) / 16;
     const bool merged = a.mode == kLogits;  // the head kernel: the only one with the argmax epilogue
-    if (!merged && a.mat.type != 7) {
-        if (a.mat.type == 9) folded<9>(a, n_rg, n_tt, stream);
-        else if (a.mat.type == 11) folded<11>(a, n_rg, n_tt, stream);
-        else folded<13>(a, n_rg, n_tt, stream);
-        return;
-    }
-    if (!merged && n_tt >= 2) {
-        // Q8_0, bound by its float step per 32-value block: two token tiles, or one while that makes about two
-        // work-groups per CU (1536 x 8960, 333 rows, 504 work-groups: 55 us on the K-split kernel, 47 here; 256 rows,
-        // 384: 39 and 45)
-        const int n_sets = (n_rg + kGemmWaves - 1) / kGemmWaves, wgs = n_sets * ((n_tt + 1) / 2);
-        const bool two = wgs >= (static_cast<int>(a.mat.cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs);
-        if (two || n_sets * n_tt >= kGemmQ8OneWgs) {
-            if (two) gemm<7, 2, 3>(a, n_rg, n_tt, stream);
-            else gemm<7, 1, 4>(a, n_rg, n_tt, stream);
+    int tpw = std::min(n_tt, kWideTpw);
+    if (merged) {
+        while (tpw > 1 && n_rg * ((n_tt + tpw - 1) / tpw) < kWideMinWgs) --tpw;
+    } else {
+        const MmRoute r = mm_route(a.mat.type, a.mat.rows, a.mat.cols, a.n_tok);
+        if (r.kernel != MmKernel::kWide) {
+            if (r.kernel == MmKernel::kStream) {
+                const dim3 g(((n_rg + kWideQ4kWaves - 1) / kWideQ4kWaves + 7) / 8 * 8), b(kWideQ4kWaves * kWave);
+                if (r.tiles == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg, 2);
+                else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg, 1);
+            } else if (a.mat.type == 7) {
+                if (r.tiles == 2) gemm<7, 2, 3>(a, n_rg, n_tt, stream);
+                else gemm<7, 1, 4>(a, n_rg, n_tt, stream);
+            } else if (a.mat.type == 9) folded<9>(a, r, n_rg, n_tt, stream);
+            else if (a.mat.type == 11) folded<11>(a, r, n_rg, n_tt, stream);
+            else folded<13>(a, r, n_rg, n_tt, stream);
             check(hipGetLastError(), "wide matmul launch");
             return;
         }
+        tpw = r.tiles;
     }
-    // as many token tiles per work-group as still leave kWideMinWgs work-groups
-    int tpw = min(n_tt, kWideTpw);
-    while (tpw > 1 && n_rg * ((n_tt + tpw - 1) / tpw) < kWideMinWgs) --tpw;
     // the head: row groups per work-group so that about kWideLogitsWgs work-groups merge their argmax
     const int rpw = a.mode == kLogits ? std::max(1, n_rg / kWideLogitsWgs) : 1;
     const int grid = (n_rg + 8 * rpw - 1) / (8 * rpw) * 8 * ((n_tt + tpw - 1) / tpw);

@@ -193,6 +193,16 @@ int32_t wide_min_rows(uint32_t type);
 // 16-token tiles per work-group; every row's result equals launch_gemv's for
 // that row alone. All modes.
 void launch_gemv_wide(const GemvArgs& a, hipStream_t stream);
+// The kernel launch_gemv_wide runs a layer matrix's step on, with the 16-row groups and 16-token tiles of a
+// work-group: Q4_K weights streamed from HBM (k_mm_wide_q4k), the long-step matmul (k_mm_gemm), the folded tiles with
+// K split over the waves (k_mm_fold), one row group per work-group (k_mm_wide).
+enum class MmKernel { kStream, kGemm, kFold, kWide };
+struct MmRoute {
+    MmKernel kernel;
+    int32_t groups;
+    int32_t tiles;
+};
+MmRoute mm_route(uint32_t type, uint32_t rows, uint32_t cols, int32_t n_tok);
 // Split-K causal GQA flash attention over the f16 caches of the step's
 // sequences. Every (row, head, split) writes its (max, sum, unnormalized
 // output) to `partial` (split stride `splits`); launch_attention_merge

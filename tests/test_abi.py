@@ -75,6 +75,15 @@ def test_weight_tile_layout_cpp_tests():
     assert "tile tests passed" in r.stdout
 
 
+def test_matmul_route_cpp_tests():
+    """Which matmul kernel a step takes, over all formats and a grid of matrix sizes and row counts."""
+    exe = os.path.join(ROOT, "tests", "cpp", "route_test")
+    subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "cpp")], check=True, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "route tests passed" in r.stdout
+
+
 def test_engine_creation_fails_loudly_without_a_gpu():
     import torch
 
