@@ -4178,7 +4178,7 @@ int32_t wide_min_rows(uint32_t type) { return wide_matmul_supported(type) ? kWid
 // (7B Q4_K down, 56 row sets: 160 rows 79 us against 83, 256 rows 109 against 86), unless K is so short that its
 // eight waves have no two tiles each (2048 x 1536 Q6_K, 256 rows: 12.7 against 10.4).
 constexpr int kCus = 256;
-constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192, kGemmQ8OneWgs = 480;
+constexpr int kGemmMinWgs = 384, kGemmShortWgs = 192;
 constexpr int kGemmFillWgs = 1024;  // four waves per SIMD everywhere
 constexpr int kGemmShortTiles = 8;
 
@@ -4206,14 +4206,20 @@ MmRoute mm_route(uint32_t type, uint32_t rows, uint32_t cols, int32_t n_tok) {
     auto wgs = [&](int tp) { return n_sets * ((n_tt + tp - 1) / tp); };
     const int two_wgs = static_cast<int>(cols) <= 256 * kGemmShortTiles ? kGemmShortWgs : kGemmMinWgs;
     if (type == 7) {
-        // Q8_0, bound by its float step per 32-value block: two token tiles, or one while that makes about two
-        // work-groups per CU (1536 x 8960, 333 rows, 504 work-groups: 55 us on the K-split kernel, 47 here; 256 rows,
-        // 384: 39 and 45)
         if (n_tt >= 2 && wgs(2) >= two_wgs) return {MmKernel::kGemm, kGemmWaves, 2};
-        if (n_tt >= 2 && wgs(1) >= kGemmQ8OneWgs) return {MmKernel::kGemm, kGemmWaves, 1};
         // as many token tiles per work-group as still leave kWideMinWgs work-groups
         int tiles = std::min(n_tt, kWideTpw);
         while (tiles > 1 && n_rg * ((n_tt + tiles - 1) / tiles) < kWideMinWgs) --tiles;
+        // Q8_0 is bound by its float step per 32-value block. On grids too small for two token tiles the one-tile
+        // long-step form takes about 1.15 us of latency per K tile and 0.15 us more per work-group of the busiest CU,
+        // the K-split form 0.3 us per K tile and work-group and 5 us for its cross-wave sums (fitted to 21 matrices,
+        // 33..2048 rows). 1536 x 8960, 333 rows: 47 us against 55, 256 rows 47 and 37; 4608 x 3584, 100 rows: 20.4 and
+        // 27.9; 5120 x 27648, 100 rows: 181 and 167.
+        auto per_cu = [](int n) { return (n + kCus - 1) / kCus; };
+        const int nb = static_cast<int>(cols) / 256, split_wgs = n_rg * ((n_tt + tiles - 1) / tiles);
+        if (tiles == 2 && nb * (115 + 15 * per_cu(wgs(1))) < nb * 30 * per_cu(split_wgs) + 500) {
+            return {MmKernel::kGemm, kGemmWaves, 1};
+        }
         return {MmKernel::kWide, 1, tiles};
     }
     // one or two token tiles against many row groups stream the weights from HBM

@@ -44,6 +44,19 @@ int main() {
             }
         }
     }
+    // Q8_0 on grids too small for two token tiles: the faster of the two forms, as measured (us)
+    struct {
+        int rows, cols, n;
+        double one_tile, split;
+    } const q8[] = {{5120, 27648, 96, 164, 141}, {5120, 27648, 128, 188, 173}, {5120, 13824, 96, 81.0, 73.3},
+                    {5120, 13824, 113, 94.4, 86.4}, {4096, 12288, 128, 78.2, 67.0}, {4096, 12288, 64, 71.1, 38.5},
+                    {3584, 18944, 100, 107.5, 92.5}, {1536, 8960, 256, 46.7, 37.6}, {1536, 8960, 333, 47, 55},
+                    {4608, 3584, 100, 20.4, 27.9}, {4608, 3584, 160, 25.5, 33.1}, {3584, 3584, 144, 20.3, 28.1},
+                    {4096, 4096, 128, 22.9, 25.8}, {10240, 2560, 48, 18.7, 25.2}};
+    for (const auto& m : q8) {
+        const MmRoute r = mm_route(7, m.rows, m.cols, m.n);
+        expect((r.kernel == MmKernel::kGemm && r.tiles == 1) == (m.one_tile < m.split), "the slower Q8_0 form", 7, m.rows, m.cols, m.n);
+    }
     if (failures == 0) std::printf("route tests passed\n");
     return failures == 0 ? 0 : 1;
 }
