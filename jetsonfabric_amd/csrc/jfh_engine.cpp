@@ -651,7 +651,7 @@ void Engine::timed(const std::string& label, double bytes, F&& fn) {
     gpu::set_launch_events(nullptr, nullptr);
 }
 
-void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits) {
+void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits, bool whole_keys) {
     const ModelParams& p = params_;
     const int32_t H = static_cast<int32_t>(p.n_embd), F = static_cast<int32_t>(p.n_ff);
     const int32_t Hq = static_cast<int32_t>(p.n_head * p.head_dim);
@@ -697,8 +697,6 @@ void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_ou
     };
     // attention split slots this step shape can fill (a prefill chunk: few long splits)
     const int32_t slots = gpu::attention_slots(splits_, attn_capacity_, n_rows, n_seq);
-    const bool whole_keys = gpu::attention_prefill_supported(n_rows, n_seq, static_cast<int32_t>(p.n_head),
-                                                             static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim));
     // l: the resident layer (its slot in the sessions' caches)
     for (uint32_t l = 0; l < layers_.size(); ++l) {
         const Layer& L = layers_[l];
@@ -1029,9 +1027,12 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
         metrics->attention_matrix_cores = p.head_dim == 64 || p.head_dim == 128;
         ++metrics->steps;
     }
+    const bool whole_keys = gpu::attention_prefill_supported(
+        rows, sd.n_seq, static_cast<int32_t>(p.n_head), static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim),
+        sd.seqs[0].pos0 + sd.seqs[0].len);
     // a long chunk's kernels outlast their launches: no graph is captured for its row count
     if (options_.use_graphs && rows <= gpu::kMaxRows) {
-        const uint64_t key = (static_cast<uint64_t>(rows) << 40) | (static_cast<uint64_t>(max_len) << 32) |
+        const uint64_t key = (whole_keys ? uint64_t{1} << 63 : 0) | (static_cast<uint64_t>(rows) << 40) | (static_cast<uint64_t>(max_len) << 32) |
                              (static_cast<uint64_t>(steps.size()) << 16) | (static_cast<uint64_t>(outs) << 1) |
                              (store ? 1u : 0u);
         auto it = graphs_.find(key);
@@ -1040,7 +1041,7 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
             hipGraph_t graph = nullptr;
             hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
             try {
-                record(rows, max_len, static_cast<int32_t>(steps.size()), outs, store);
+                record(rows, max_len, static_cast<int32_t>(steps.size()), outs, store, whole_keys);
             } catch (...) {
                 (void) hipStreamEndCapture(stream_, &graph);
                 if (graph) (void) hipGraphDestroy(graph);
@@ -1061,7 +1062,7 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
         hip_check(hipGraphLaunch(it->second, stream_), "launch step graph");
     } else {
         if (metrics) hip_check(hipEventRecord(ev_begin_, stream_), "time step");
-        record(rows, max_len, static_cast<int32_t>(steps.size()), outs, store);
+        record(rows, max_len, static_cast<int32_t>(steps.size()), outs, store, whole_keys);
     }
     if (metrics) hip_check(hipEventRecord(ev_compute_, stream_), "time step");
     if (outs > 0) {

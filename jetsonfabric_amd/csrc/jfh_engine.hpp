@@ -260,7 +260,7 @@ private:
     const float* upload_f32(const TensorView& t);
     void ensure_capacity(uint32_t capacity);
     uint32_t balanced_chunk(uint32_t n) const;
-    void record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits);
+    void record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits, bool whole_keys);
     template <typename F>
     void timed(const std::string& label, double bytes, F&& fn);
 
@@ -315,7 +315,7 @@ private:
     // normalized int8 rows of wide steps (the QKV and gate/up inputs)
     gpu::Act8 xq_norm_;
 
-    // captured step graphs keyed by (rows, seqs, outs, store_logits)
+    // captured step graphs keyed by (rows, seqs, outs, store_logits, attention without key splits)
     std::map<uint64_t, hipGraphExec_t> graphs_;
     std::vector<int32_t> end_tokens_;
     mutable std::mutex mutex_;

@@ -4323,9 +4323,6 @@ void launch_embed(const DMat& table, const StepDev* step, float* h, int32_t n_ro
     check(hipGetLastError(), "embed launch");
 }
 
-// Fewest work-groups of 64 query rows from which a prefill chunk runs without key splits.
-constexpr int kPrefillAttnMinWgs = 128;
-
 int32_t attention_max_rows(int32_t head_dim) {
     // the matrix-core kernel takes any number of 16-row groups; the generic one up to kMaxAttnQGroups groups of 8
     return (head_dim == 128 || head_dim == 64) ? kMaxRows * 64 : kMaxAttnQGroups * kAttnQPW;
@@ -4387,10 +4384,19 @@ void launch_attention(const float* q, const StepDev* step, int32_t max_len, int3
     check(hipGetLastError(), "attention launch");
 }
 
-bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim) {
+// Without key splits a step takes the time of one work-group's walk over all keys (35 ns per key at head dim 128, 22
+// at 64) however few CUs have one; with splits it goes with the work-groups (0.23 and 0.11 ns per key and 64 query rows;
+// one head per kv head 0.19 and 0.09) plus the empty and merged splits of short sequences. Measured, us with splits and
+// without: 40 heads / 8 kv heads x 128, 204 rows (128 work-groups) 26 / 23.5 at 64 positions, 161 / 163 at 4096,
+// 716 / 872 at 24576; 256 rows (160) 197 / 157 at 4096, 884 / 838 at 24576; 32 / 32 x 128, 200 rows 57 / 56 at 1024,
+// 136 / 161 at 4096; 64 / 8 x 64, 128 rows 29 / 25 at 512, 81 / 101 at 4096, 192 rows 498 / 536 at 24576.
+bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
+                                 int32_t n_keys) {
     if (n_seq != 1 || n_rows <= kQuadGroupRows || (head_dim != 128 && head_dim != 64)) return false;
-    const int qblocks = (n_head / n_head_kv * n_rows + 4 * kAttnRows - 1) / (4 * kAttnRows);
-    return n_rows > kMaxRows || qblocks * n_head_kv >= kPrefillAttnMinWgs;
+    if (n_rows > kMaxRows) return true;
+    const int G = n_head / n_head_kv, wgs = (G * n_rows + 4 * kAttnRows - 1) / (4 * kAttnRows) * n_head_kv;
+    if (n_keys <= (head_dim == 128 ? 1280 : 768)) return wgs >= 128;
+    return wgs >= (head_dim == 64 ? 256 : G >= 4 ? 160 : 192);
 }
 
 void launch_attention_prefill(const float* q, const StepDev* step, int32_t n_rows, int32_t layer, int32_t n_head,

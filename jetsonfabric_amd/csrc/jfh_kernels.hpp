@@ -213,9 +213,10 @@ void launch_attention(const float* q, const StepDev* step, int32_t max_len, int3
                       int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t splits, float* partial,
                       hipStream_t stream, int32_t slots = 0);
 // Attention of one sequence's n_rows rows (a prefill chunk; head dims 64 and 128) without key splits: writes the
-// attention output rows to out [row][n_head * head_dim]. attention_prefill_supported: whether a step takes it (every
-// chunk of more than kMaxRows rows does; the split partials hold kMaxRows rows).
-bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim);
+// attention output rows to out [row][n_head * head_dim]. attention_prefill_supported: whether a step whose sequence then
+// holds n_keys positions takes it (every chunk of more than kMaxRows rows does; the split partials hold kMaxRows rows).
+bool attention_prefill_supported(int32_t n_rows, int32_t n_seq, int32_t n_head, int32_t n_head_kv, int32_t head_dim,
+                                 int32_t n_keys);
 void launch_attention_prefill(const float* q, const StepDev* step, int32_t n_rows, int32_t layer, int32_t n_head,
                               int32_t n_head_kv, int32_t head_dim, float* out, hipStream_t stream);
 // Merges the splits of every (row, head) into out[row][n_head * head_dim]

@@ -1,6 +1,7 @@
 // Host check of which kernel a layer matrix's step takes (gpu::mm_route): no work-group is given a token tile that the
 // step does not have, and a K-split step takes two token tiles per work-group only where the busiest CU's work-groups
-// then take less time (measured cost of a two-tile work-group against a one-tile one: Q6_K 1.45, others 1.7-1.8).
+// then take less time (measured cost of a two-tile work-group against a one-tile one: Q6_K 1.45, others 1.7-1.8). And
+// which attention a step takes, against measured times.
 #include "jfh_kernels.hpp"
 
 #include <cstdio>
@@ -56,6 +57,25 @@ int main() {
     for (const auto& m : q8) {
         const MmRoute r = mm_route(7, m.rows, m.cols, m.n);
         expect((r.kernel == MmKernel::kGemm && r.tiles == 1) == (m.one_tile < m.split), "the slower Q8_0 form", 7, m.rows, m.cols, m.n);
+    }
+    // attention of one sequence's step at a position: with key splits and without, as measured (us)
+    struct {
+        int heads, kv, dim, pos, rows;
+        double split, whole;
+    } const attn[] = {{40, 8, 128, 64, 217, 33.7, 23.7},   {40, 8, 128, 1024, 230, 71.9, 57.5},
+                      {40, 8, 128, 8192, 204, 288, 303},   {40, 8, 128, 24576, 204, 716, 872},
+                      {40, 8, 128, 24576, 230, 800, 880},  {40, 8, 128, 24576, 256, 884, 838},
+                      {32, 32, 128, 1024, 200, 57.0, 55.9}, {32, 32, 128, 2048, 200, 81.5, 90.8},
+                      {32, 32, 128, 24576, 200, 595, 869}, {64, 8, 128, 4096, 192, 233, 155},
+                      {64, 8, 128, 24576, 136, 759, 832},  {64, 8, 64, 512, 128, 29.2, 25.4},
+                      {64, 8, 64, 2048, 128, 50.7, 58.0},  {64, 8, 64, 8192, 160, 164, 189},
+                      {64, 8, 64, 24576, 192, 498, 536},   {32, 32, 64, 4096, 200, 69.2, 109}};
+    for (const auto& m : attn) {
+        const bool whole = jfh::gpu::attention_prefill_supported(m.rows, 1, m.heads, m.kv, m.dim, m.pos + m.rows);
+        if (whole != (m.whole < m.split)) {
+            ++failures;
+            std::printf("FAIL: the slower attention: %d / %d heads x %d, %d rows at %d\n", m.heads, m.kv, m.dim, m.rows, m.pos);
+        }
     }
     if (failures == 0) std::printf("route tests passed\n");
     return failures == 0 ? 0 : 1;
