@@ -1102,15 +1102,15 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
 
 PrefillMetrics Engine::last_prefill_metrics() { return t_last_prefill; }
 
-uint64_t Engine::scratch_bytes_per_row() const {
+uint64_t Engine::scratch_bytes(uint32_t rows) const {
     const ModelParams& p = params_;
     const uint64_t H = p.n_embd, Hq = static_cast<uint64_t>(p.n_head) * p.head_dim, F = p.n_ff;
-    auto act8 = [](const gpu::Act8& a) { return a.q ? a.K + a.K / 32 * 4 + a.K / 16 * 2 : 0; };
-    uint64_t b = (H + 2 * Hq + F) * sizeof(float) + act8(xq_attn_) + act8(xq_ffn_) + act8(xq_norm_);
-    b += gpu::attention_partial_floats(1, static_cast<int32_t>(p.n_head), static_cast<int32_t>(p.head_dim), splits_) *
-         sizeof(float);
-    if (logits_) b += static_cast<uint64_t>(p.n_vocab) * sizeof(float);
-    return b;
+    auto act8 = [](const gpu::Act8& a) -> uint64_t { return a.q ? a.K + a.K / 32 * 4 + a.K / 16 * 2 : 0; };
+    const uint64_t row = (H + 2 * Hq + F) * sizeof(float) + act8(xq_attn_) + act8(xq_ffn_) + act8(xq_norm_);
+    uint64_t step_row = gpu::attention_partial_floats(1, static_cast<int32_t>(p.n_head), static_cast<int32_t>(p.head_dim),
+                                                      splits_) * sizeof(float);
+    if (logits_) step_row += static_cast<uint64_t>(p.n_vocab) * sizeof(float);
+    return rows * row + std::min<uint64_t>(rows, gpu::kMaxRows) * step_row;
 }
 
 BufferMetrics Engine::buffer_metrics(uint32_t capacity, uint32_t prompt_tokens, const PrefillMetrics& prefill) const {
@@ -1118,8 +1118,9 @@ BufferMetrics Engine::buffer_metrics(uint32_t capacity, uint32_t prompt_tokens, 
     BufferMetrics m;
     const uint64_t stride = (std::max<uint32_t>(capacity, 16) + 15) / 16 * 16;  // as Session allocates
     m.kv_cache_bytes = 2ull * resident_layers() * p.n_head_kv * stride * p.head_dim * sizeof(uint16_t);
-    m.prefill_scratch_bytes = scratch_bytes_per_row() * std::min<uint64_t>(prefill_chunk_, std::max<uint32_t>(1, prompt_tokens));
-    m.decode_scratch_bytes = scratch_bytes_per_row();
+    const uint32_t prompt = std::max<uint32_t>(1, prompt_tokens);
+    m.prefill_scratch_bytes = scratch_bytes(std::min(prompt, balanced_chunk(prompt)));
+    m.decode_scratch_bytes = scratch_bytes(1);
     m.prefill_host_input_bytes = prefill.host_input_bytes;
     return m;
 }

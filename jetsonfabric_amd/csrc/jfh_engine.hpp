@@ -53,7 +53,7 @@ struct PrefillMetrics {
 // Device buffers a generation uses (ExecutionBufferMetrics, native_inference.hpp:80-85).
 struct BufferMetrics {
     uint64_t kv_cache_bytes = 0;          // the session's F16 K/V cache
-    uint64_t prefill_scratch_bytes = 0;   // workspace rows of one prefill chunk
+    uint64_t prefill_scratch_bytes = 0;   // workspace of the longest prefill chunk's rows
     uint64_t decode_scratch_bytes = 0;    // workspace of one decode row
     uint64_t prefill_host_input_bytes = 0;
 };
@@ -216,9 +216,10 @@ public:
 
     uint32_t max_prefill_chunk() const { return prefill_chunk_; }
 
-    // Workspace bytes one token row of a step uses (residual, queries,
-    // attention and SwiGLU outputs, their int8 copies, attention partials).
-    uint64_t scratch_bytes_per_row() const;
+    // Workspace bytes `rows` token rows use: residual, queries, attention and
+    // SwiGLU outputs and their int8 copies; logits and attention partials for
+    // the rows of a step (kMaxRows) at most.
+    uint64_t scratch_bytes(uint32_t rows) const;
     // Buffer metrics of a session of `capacity` positions whose prefill ran
     // `prompt_tokens` tokens with the given metrics.
     BufferMetrics buffer_metrics(uint32_t capacity, uint32_t prompt_tokens, const PrefillMetrics& prefill) const;

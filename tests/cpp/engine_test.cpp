@@ -1,0 +1,66 @@
+// Host-side tests of the engine on a device in host memory (fake_device.hpp): what a prefill reports and how it is cut
+// into chunks, the buffers of sessions, and allocations that fail.
+#include "fake_device.hpp"
+
+#include <memory>
+#include <string>
+#include <vector>
+
+using namespace jfh;
+
+namespace {
+
+int failures = 0;
+
+void expect(bool ok, const std::string& what) {
+    if (ok) return;
+    ++failures;
+    std::printf("FAIL: %s\n", what.c_str());
+}
+
+constexpr uint32_t kVocab = 512, kCtx = 8192, kLayers = 2, kEmbd = 512, kFf = 768, kHeads = 8, kKvHeads = 2, kDim = 64;
+
+std::unique_ptr<Engine> engine(uint32_t layer_start = 0, uint32_t layer_end = kLayers) {
+    SynthSpec spec;
+    spec.params = {kLayers, kEmbd, kFf, kHeads, kKvHeads, kCtx, kVocab, kDim, 1.0e6F, 1.0e-6F};
+    const auto model = HostModel::synthesize(spec);
+    if (layer_start == 0 && layer_end == kLayers) return std::make_unique<Engine>(*model, EngineOptions{});
+    return std::make_unique<Engine>(*model->slice(layer_start, layer_end), EngineOptions{});
+}
+
+std::vector<int32_t> prompt(uint32_t n) {
+    std::vector<int32_t> ids(n);
+    for (uint32_t i = 0; i < n; ++i) ids[i] = static_cast<int32_t>(i * 7 % kVocab);
+    return ids;
+}
+
+// The workspace a prefill reports: what its longest chunk's rows take, with logits rows and attention partials for
+// the rows of a step only.
+void test_prefill_scratch() {
+    const auto e = engine();
+    auto act8 = [](uint64_t K) { return K + K / 32 * 4 + K / 16 * 2; };
+    constexpr uint64_t F = 4;
+    const uint64_t row = (kEmbd + 2 * kHeads * kDim + kFf) * F + act8(kHeads * kDim) + act8(kFf) + act8(kEmbd);
+    for (uint32_t n : {1u, 100u, 256u, 300u, 1500u, 2048u, 2200u, 5000u}) {
+        const auto s = e->create_session(n);
+        e->prefill(*s, prompt(n).data(), n, nullptr);
+        const uint32_t chunks = s->prefill_metrics().steps;
+        const BufferMetrics m = e->buffer_metrics(n, n, s->prefill_metrics());
+        const uint64_t wide = m.decode_scratch_bytes - row;  // a row's logits and attention partials
+        // the longest of about equally long chunks
+        const uint64_t longest = chunks == 1 ? n : ((n + chunks - 1) / chunks + 127) / 128 * 128;
+        expect(wide >= kVocab * F && wide <= kVocab * F + 32 * kHeads * (kDim + 2) * F, "decode scratch of a row");
+        expect(m.prefill_scratch_bytes == longest * row + std::min<uint64_t>(longest, 256) * wide,
+               "prefill scratch of " + std::to_string(n) + " tokens: " + std::to_string(m.prefill_scratch_bytes));
+        expect(m.prefill_scratch_bytes <= fake::live_bytes, "prefill scratch exceeds what is allocated");
+    }
+}
+
+}  // namespace
+
+int main() {
+    test_prefill_scratch();
+    failures += fake::faults;
+    if (failures == 0) std::printf("engine tests passed\n");
+    return failures == 0 ? 0 : 1;
+}

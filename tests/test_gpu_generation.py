@@ -125,7 +125,13 @@ def test_generation_metrics(engine):
         # the session the runner opened: capacity prompt + n rounded up to 16 positions, F16 K and V
         stride = -(-(len(prompt) + n) // 16) * 16
         assert b["kv_cache_bytes"] == 2 * CFG.n_layer * CFG.n_head_kv * stride * (CFG.n_embd // CFG.n_head) * 2
-        assert b["prefill_scratch_bytes"] == min(engine.prefill_chunk, len(prompt)) * b["decode_scratch_bytes"] > 0
+        # every row of the chunk: residual, queries, attention and SwiGLU outputs and their int8 copies; logits and
+        # attention partials (the rest of what a decode row takes) for the 256 rows of a step at most
+        def act8(k):
+            return k + k // 32 * 4 + k // 16 * 2
+        row = (3 * CFG.n_embd + CFG.n_ff) * 4 + 2 * act8(CFG.n_embd) + act8(CFG.n_ff)
+        assert b["decode_scratch_bytes"] > row + CFG.n_vocab * 4
+        assert b["prefill_scratch_bytes"] == 300 * row + 256 * (b["decode_scratch_bytes"] - row)
     # the second run replays the step graphs the first one captured
     assert again.prefill["plan_reused"] and again.prefill["planning_ms"] == 0.0
     assert first.sampled_tokens == again.sampled_tokens
