@@ -47,7 +47,7 @@ bool quantized(uint32_t type) { return type == kQ4_K || type == kQ6_K || type ==
 thread_local PrefillMetrics t_last_prefill;
 
 // ------------------------------------------------------------------ cache buffers
-void* CachePool::take(size_t bytes, size_t& size) {
+CachePool::Buffer CachePool::take(size_t bytes) {
     constexpr size_t kUnit = size_t{1} << 20;
     const size_t want = (bytes + kUnit - 1) / kUnit * kUnit;
     {
@@ -62,30 +62,40 @@ void* CachePool::take(size_t bytes, size_t& size) {
             const Buffer b = free_[best];
             free_.erase(free_.begin() + static_cast<std::ptrdiff_t>(best));
             held_ -= b.size;
-            size = b.size;
-            return b.p;
+            return b;
         }
     }
-    void* p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
+    Buffer b;
+    b.size = want;
+    if (hipMalloc(&b.p, want) != hipSuccess) {
         (void) hipGetLastError();
         drain();
-        if (hipMalloc(&p, want) != hipSuccess) return nullptr;
+        if (hipMalloc(&b.p, want) != hipSuccess) return {};
     }
-    size = want;
-    return p;
+    if (hipEventCreate(&b.clear_begin) != hipSuccess || hipEventCreate(&b.clear_end) != hipSuccess) {
+        release(b);
+        return {};
+    }
+    return b;
 }
 
-void CachePool::put(void* p, size_t size) {
-    if (p == nullptr) return;
+void CachePool::release(const Buffer& b) {
+    (void) hipFree(b.p);
+    for (hipEvent_t e : {b.clear_begin, b.clear_end}) {
+        if (e) (void) hipEventDestroy(e);
+    }
+}
+
+void CachePool::put(const Buffer& b) {
+    if (b.p == nullptr) return;
     std::vector<Buffer> out;
     {
         std::lock_guard lock(mutex_);
-        if (closed_ || size > kBytes) {
-            out.push_back({p, size});
+        if (closed_ || b.size > kBytes) {
+            out.push_back(b);
         } else {
-            free_.push_back({p, size});
-            held_ += size;
+            free_.push_back(b);
+            held_ += b.size;
             while (free_.size() > kBuffers || held_ > kBytes) {  // the longest kept ones go first
                 held_ -= free_.front().size;
                 out.push_back(free_.front());
@@ -93,7 +103,7 @@ void CachePool::put(void* p, size_t size) {
             }
         }
     }
-    for (const Buffer& b : out) (void) hipFree(b.p);
+    for (const Buffer& o : out) release(o);
 }
 
 void CachePool::drain() {
@@ -103,7 +113,7 @@ void CachePool::drain() {
         out.swap(free_);
         held_ = 0;
     }
-    for (const Buffer& b : out) (void) hipFree(b.p);
+    for (const Buffer& b : out) release(b);
 }
 
 void CachePool::close() {
@@ -121,18 +131,27 @@ Session::Session(Engine* engine, uint32_t capacity)
     const size_t elems = static_cast<size_t>(engine->resident_layers()) * p.n_head_kv * stride_ * p.head_dim;
     kv_bytes_ = 2 * elems * sizeof(uint16_t);
     pool_ = engine->pool_;
-    k_ = static_cast<uint16_t*>(pool_->take(kv_bytes_, buffer_bytes_));
-    if (k_ == nullptr) fail(Status::OutOfMemory, "allocate K and V cache");
+    buffer_ = pool_->take(kv_bytes_);
+    if (buffer_.p == nullptr) fail(Status::OutOfMemory, "allocate K and V cache");
+    k_ = static_cast<uint16_t*>(buffer_.p);
     v_ = k_ + elems;
     // every use of the cache is ordered behind this on the engine's stream
-    const hipError_t e = hipMemsetAsync(k_, 0, kv_bytes_, engine->stream());
+    hipError_t e = hipEventRecord(buffer_.clear_begin, engine->stream());
+    if (e == hipSuccess) e = hipMemsetAsync(k_, 0, kv_bytes_, engine->stream());
+    if (e == hipSuccess) e = hipEventRecord(buffer_.clear_end, engine->stream());
     if (e != hipSuccess) {
-        pool_->put(k_, buffer_bytes_);
+        pool_->put(buffer_);
         hip_check(e, "clear KV cache");
     }
 }
 
-Session::~Session() { pool_->put(k_, buffer_bytes_); }
+Session::~Session() { pool_->put(buffer_); }
+
+double Session::clear_ms() const {
+    float ms = 0.0F;
+    hip_check(hipEventElapsedTime(&ms, buffer_.clear_begin, buffer_.clear_end), "cache clearing time");
+    return ms;
+}
 
 void Session::rollback(uint32_t n) {
     // qwen2_architecture.cpp:818-823: only the decoded suffix can be removed;
@@ -1152,6 +1171,7 @@ int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* lo
         done += len;
     }
     s.prefill_position_ = n;
+    m.allocation_ms += s.clear_ms();
     s.prefill_metrics_ = m;
     t_last_prefill = m;
     return token;
@@ -1190,6 +1210,7 @@ int32_t Engine::stage_prefill(Session& s, const int32_t* tokens, const float* ac
         done += len;
     }
     s.prefill_position_ = n;
+    m.allocation_ms += s.clear_ms();
     s.prefill_metrics_ = m;
     t_last_prefill = m;
     return token;

@@ -66,18 +66,20 @@ class CachePool {
 public:
     static constexpr size_t kBytes = size_t{256} << 20;
     static constexpr size_t kBuffers = 8;
+    struct Buffer {
+        void* p = nullptr;
+        size_t size = 0;
+        hipEvent_t clear_begin = nullptr, clear_end = nullptr;  // around its last clearing
+    };
     ~CachePool() { close(); }
-    // A buffer of at least `bytes` (its size is stored in `size`), nullptr when the device has no memory left.
-    void* take(size_t bytes, size_t& size);
-    void put(void* p, size_t size);
+    // A buffer of at least `bytes`, p == nullptr when the device has no memory left.
+    Buffer take(size_t bytes);
+    void put(const Buffer& b);
     void drain();
     void close();  // drains; buffers put back later are freed
 
 private:
-    struct Buffer {
-        void* p;
-        size_t size;
-    };
+    static void release(const Buffer& b);
     std::mutex mutex_;
     std::vector<Buffer> free_;
     size_t held_ = 0;
@@ -101,6 +103,8 @@ public:
 private:
     friend class Engine;
     Session(Engine* engine, uint32_t capacity);
+    // Device time of the cache's clearing (once a step of the session has finished).
+    double clear_ms() const;
 
     Engine* engine_;
     uint32_t capacity_;
@@ -108,7 +112,7 @@ private:
     uint32_t position_ = 0;
     uint32_t prefill_position_ = 0;
     std::shared_ptr<CachePool> pool_;
-    size_t buffer_bytes_ = 0;  // of the buffer that holds K, then V
+    CachePool::Buffer buffer_;  // holds K, then V
     uint16_t* k_ = nullptr;  // [resident layer][kv head][stride][head_dim]
     uint16_t* v_ = nullptr;  // [resident layer][kv head][stride / 16][head_dim][16] (16-position tiles)
     uint64_t kv_bytes_ = 0;

@@ -56,9 +56,24 @@ void test_prefill_scratch() {
     }
 }
 
+// A prefill's allocation time holds the clearing of its session's cache, in a new buffer and in one kept from a closed
+// session; its compute time does not.
+void test_allocation_time() {
+    const auto e = engine();
+    for (int i = 0; i < 3; ++i) {
+        const auto s = e->create_session(3000);
+        const double clearing = 100.0 * static_cast<double>(s->kv_bytes()) / (1 << 20);
+        e->prefill(*s, prompt(2500).data(), 2500, nullptr);
+        const PrefillMetrics& m = s->prefill_metrics();
+        expect(m.allocation_ms >= 0.999 * clearing, "allocation time " + std::to_string(m.allocation_ms) + " ms, clearing " + std::to_string(clearing));
+        expect(m.compute_ms > 0.0 && m.compute_ms < 0.5 * clearing, "compute time " + std::to_string(m.compute_ms));
+    }
+}
+
 }  // namespace
 
 int main() {
+    test_allocation_time();
     test_prefill_scratch();
     failures += fake::faults;
     if (failures == 0) std::printf("engine tests passed\n");

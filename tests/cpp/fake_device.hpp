@@ -1,7 +1,7 @@
 // A device in host memory for host-side tests of the engine: the HIP runtime calls jfh_engine.cpp makes and the kernel
 // launchers of jfh_kernels.hpp. "Device" memory is host memory with known bounds, copies and fills are checked against
 // them, launches change nothing (a stage's residual rows come out as they went in) and a clock of its own stands for
-// device time: a fill takes 1 ms per MB, a launch 1 us per row.
+// device time: a fill takes 100 ms per MB, a launch 1 us per row.
 #pragma once
 
 #include "jfh_engine.hpp"
@@ -107,7 +107,7 @@ hipError_t hipMemset(void* d, int v, size_t n) {
         return hipErrorInvalidValue;
     }
     std::memset(d, v, n);
-    fake::clock_ms += static_cast<double>(n) / (1 << 20);
+    fake::clock_ms += 100.0 * static_cast<double>(n) / (1 << 20);
     return hipSuccess;
 }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
