@@ -574,23 +574,26 @@ void Engine::ensure_capacity(uint32_t capacity) {
     const uint32_t cap = std::min<uint32_t>(p.n_ctx, std::max<uint32_t>(capacity, 256));
     std::vector<float> table(static_cast<size_t>(cap) * p.head_dim);
     rope_rows(p.rope_base, p.head_dim, 0, cap, table.data());
-    if (rope_) (void) hipFree(rope_);
-    rope_ = nullptr;
+    // Captured steps hold the old table and partials. Until the new ones are in place the engine counts as sized for
+    // nothing, so that after a failed allocation the next step or session sizes it again.
+    for (auto& [key, exec] : graphs_) (void) hipGraphExecDestroy(exec);
+    graphs_.clear();
+    capacity_max_ = 0;
+    for (float** p : {&rope_, &partial_}) {
+        if (*p) (void) hipFree(*p);
+        *p = nullptr;
+    }
     hip_check(hipMalloc(&rope_, table.size() * sizeof(float)), "allocate rope table");
     hip_check(hipMemcpy(rope_, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice), "upload rope table");
     splits_ = gpu::attention_splits(static_cast<int32_t>(cap));
     attn_capacity_ = static_cast<int32_t>(cap);
     const size_t partial_floats = gpu::attention_partial_floats(gpu::kMaxRows, static_cast<int32_t>(p.n_head),
                                                                 static_cast<int32_t>(p.head_dim), splits_);
-    if (partial_) (void) hipFree(partial_);
-    partial_ = nullptr;
     if (hipMalloc(&partial_, partial_floats * sizeof(float)) != hipSuccess) {
         pool_->drain();
         hip_check(hipMalloc(&partial_, partial_floats * sizeof(float)), "allocate attention partials");
     }
     capacity_max_ = cap;
-    for (auto& [key, exec] : graphs_) (void) hipGraphExecDestroy(exec);
-    graphs_.clear();
 }
 
 std::unique_ptr<Session> Engine::create_session(uint32_t capacity) {
@@ -988,6 +991,7 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
             fail(Status::InvalidArgument, "too many rows for one sequence step");
         }
         if (static_cast<uint64_t>(rows) + st.n > row_limit) fail(Status::InvalidArgument, "too many token rows in one step");
+        ensure_capacity(s->capacity_);  // sized when the session was created, unless a later session's sizing failed
         sd.seqs[si].k = s->k_;
         sd.seqs[si].v = s->v_;
         sd.seqs[si].capacity = static_cast<int32_t>(s->stride_);

@@ -70,9 +70,43 @@ void test_allocation_time() {
     }
 }
 
+template <typename F>
+bool refused(F&& f) {
+    try {
+        f();
+    } catch (const Error&) {
+        return true;
+    }
+    return false;
+}
+
+// A session that the device has no memory for leaves the engine and its open sessions usable.
+void test_failed_capacity() {
+    for (size_t limit : {size_t{0}, size_t{100} << 10, size_t{3} << 20}) {  // refusing the rope table, the partials, the cache
+        const auto e = engine();
+        const auto s = e->create_session(300);
+        e->prefill(*s, prompt(200).data(), 200, nullptr);
+        SeqStep st;
+        const int32_t id = 3;
+        st.session = s.get();
+        st.tokens = &id;
+        st.n = 1;
+        e->forward({st}, nullptr, nullptr, nullptr);
+        fake::fail_from = (size_t{100} << 10) + limit;
+        fake::memory = fake::live_bytes + limit;
+        expect(refused([&] { (void) e->create_session(kCtx); }), "a session larger than the device's memory");
+        fake::memory = fake::fail_from = ~size_t{0};
+        e->forward({st}, nullptr, nullptr, nullptr);
+        expect(s->position() == 202, "step after a refused session");
+        const auto t = e->create_session(kCtx);
+        e->forward({st}, nullptr, nullptr, nullptr);
+    }
+}
+
 }  // namespace
 
 int main() {
+    test_failed_capacity();
     test_allocation_time();
     test_prefill_scratch();
     failures += fake::faults;

@@ -1,6 +1,7 @@
 // A device in host memory for host-side tests of the engine: the HIP runtime calls jfh_engine.cpp makes and the kernel
 // launchers of jfh_kernels.hpp. "Device" memory is host memory with known bounds, copies and fills are checked against
-// them, launches change nothing (a stage's residual rows come out as they went in) and a clock of its own stands for
+// them, launches change nothing (a stage's residual rows come out as they went in; captured ones run when their graph
+// does) and a clock of its own stands for
 // device time: a fill takes 100 ms per MB, a launch 1 us per row.
 #pragma once
 
@@ -11,9 +12,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <thread>
+#include <vector>
 
 namespace fake {
 
@@ -41,9 +44,21 @@ inline bool inside(const void* p, size_t n) {
     return a + n <= it->first + it->second;
 }
 
+// A launch: runs now, or with the graph being captured.
+inline bool capturing = false;
+using Work = std::vector<std::function<void()>>;
+inline Work captured;
+
+inline void launch(std::function<void()> work) {
+    if (capturing) captured.push_back(std::move(work));
+    else work();
+}
+
 inline void launched(double rows) {
-    std::lock_guard l(lock);
-    clock_ms += rows * 1e-3;
+    launch([rows] {
+        std::lock_guard l(lock);
+        clock_ms += rows * 1e-3;
+    });
 }
 
 }  // namespace fake
@@ -120,15 +135,30 @@ hipError_t hipStreamSynchronize(hipStream_t) {
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { ++fake::captures; return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = reinterpret_cast<hipGraph_t>(1); return hipSuccess; }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
-    *e = reinterpret_cast<hipGraphExec_t>(1);
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
+    ++fake::captures;
+    fake::capturing = true;
+    fake::captured.clear();
     return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+    fake::capturing = false;
+    *g = reinterpret_cast<hipGraph_t>(1);
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+    *e = reinterpret_cast<hipGraphExec_t>(new fake::Work(fake::captured));
+    return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+    for (const auto& work : *reinterpret_cast<fake::Work*>(e)) work();
+    return hipSuccess;
+}
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
+    delete reinterpret_cast<fake::Work*>(e);
+    return hipSuccess;
+}
 
 hipError_t hipEventCreate(hipEvent_t* e) { *e = new ihipEvent_t; return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
@@ -149,15 +179,40 @@ namespace jfh::gpu {
 
 void set_launch_events(hipEvent_t, hipEvent_t) {}
 void launch_embed(const DMat&, const StepDev*, float*, int32_t n, int32_t, unsigned long long*, int32_t, hipStream_t) { fake::launched(n); }
-void launch_gemv(const GemvArgs& a, hipStream_t) { fake::launched(a.n_tok); }
-void launch_gemv_wide(const GemvArgs& a, hipStream_t) { fake::launched(a.n_tok); }
+void launch_gemv(const GemvArgs& a, hipStream_t) {
+    fake::launched(a.n_tok);
+    if (a.mode != kQKV) return;
+    fake::launch([a] {  // reads the rows' rotations
+        std::lock_guard l(fake::lock);
+        for (int32_t t = 0; t < a.n_tok; ++t) {
+            const size_t row = static_cast<size_t>(a.qkv.head_dim) * sizeof(float);
+            if (a.qkv.rope == nullptr ||
+                !fake::inside(a.qkv.rope + static_cast<size_t>(a.qkv.step->rows[a.qkv.row0 + t].pos) * a.qkv.head_dim, row)) {
+                fake::fault("rope read");
+                return;
+            }
+        }
+    });
+}
+void launch_gemv_wide(const GemvArgs& a, hipStream_t s) { launch_gemv(a, s); }
 void launch_quantize(const float*, int32_t, int32_t n, const Act8&, hipStream_t) { fake::launched(n); }
 void launch_quantize_norm(const float*, int32_t, const int32_t*, const float*, float, int32_t n, const Act8&, hipStream_t) { fake::launched(n); }
-void launch_attention(const float*, const StepDev* st, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, float*, hipStream_t, int32_t) {
-    fake::step_rows = static_cast<uint32_t>(st->n_rows);
+size_t attention_partial_floats(int32_t rows, int32_t n_head, int32_t head_dim, int32_t splits) {
+    return static_cast<size_t>(rows) * n_head * splits * (head_dim + 2);
+}
+void launch_attention(const float*, const StepDev* st, int32_t, int32_t, int32_t, int32_t n_head, int32_t, int32_t head_dim,
+                      int32_t splits, float* partial, hipStream_t, int32_t) {
+    fake::launch([=] {
+        std::lock_guard l(fake::lock);
+        if (partial == nullptr ||
+            !fake::inside(partial, attention_partial_floats(st->n_rows, n_head, head_dim, splits) * sizeof(float))) {
+            fake::fault("attention partials");
+        }
+        fake::step_rows = static_cast<uint32_t>(st->n_rows);
+    });
 }
 void launch_attention_prefill(const float*, const StepDev*, int32_t n, int32_t, int32_t, int32_t, int32_t, float*, hipStream_t) {
-    fake::step_rows = static_cast<uint32_t>(n);
+    fake::launch([n] { fake::step_rows = static_cast<uint32_t>(n); });
 }
 void launch_attention_merge(const float*, const StepDev*, int32_t n, int32_t, int32_t, int32_t, float*, const Act8&, hipStream_t, int32_t) { fake::launched(n); }
 void launch_finish(unsigned long long*, const StepDev*, int32_t, StepOut*, hipStream_t) {}
@@ -167,9 +222,6 @@ int32_t wide_min_rows(uint32_t) { return 9; }
 int32_t attention_splits(int32_t capacity) { return std::min(32, (capacity + 63) / 64); }
 int32_t attention_slots(int32_t splits, int32_t, int32_t, int32_t) { return splits; }
 int32_t attention_max_rows(int32_t) { return kMaxRows * 64; }
-size_t attention_partial_floats(int32_t rows, int32_t n_head, int32_t head_dim, int32_t splits) {
-    return static_cast<size_t>(rows) * n_head * splits * (head_dim + 2);
-}
 bool attention_prefill_supported(int32_t n_rows, int32_t, int32_t, int32_t, int32_t, int32_t) { return n_rows > kMaxRows; }
 void scratch_setup(int) {}
 void* scratch_address(int) { return nullptr; }
