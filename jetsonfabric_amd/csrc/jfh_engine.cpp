@@ -47,6 +47,44 @@ bool quantized(uint32_t type) { return type == kQ4_K || type == kQ6_K || type ==
 thread_local PrefillMetrics t_last_prefill;
 
 // ------------------------------------------------------------------ cache buffers
+namespace {
+
+// Every engine's pool. The lock is held while one drains, so that none goes away meanwhile.
+struct Pools {
+    std::mutex mutex;
+    std::vector<CachePool*> list;
+};
+
+Pools& pools() {
+    static Pools* p = new Pools;  // never destroyed: a session may be closed while the process ends
+    return *p;
+}
+
+}  // namespace
+
+CachePool::CachePool() {
+    std::lock_guard lock(pools().mutex);
+    pools().list.push_back(this);
+}
+
+CachePool::~CachePool() {
+    {
+        std::lock_guard lock(pools().mutex);
+        std::erase(pools().list, this);
+    }
+    close();
+}
+
+hipError_t CachePool::allocate(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
+    (void) hipGetLastError();
+    {
+        std::lock_guard lock(pools().mutex);
+        for (CachePool* pool : pools().list) pool->drain();
+    }
+    return hipMalloc(p, bytes);
+}
+
 CachePool::Buffer CachePool::take(size_t bytes) {
     constexpr size_t kUnit = size_t{1} << 20;
     const size_t want = (bytes + kUnit - 1) / kUnit * kUnit;
@@ -67,11 +105,7 @@ CachePool::Buffer CachePool::take(size_t bytes) {
     }
     Buffer b;
     b.size = want;
-    if (hipMalloc(&b.p, want) != hipSuccess) {
-        (void) hipGetLastError();
-        drain();
-        if (hipMalloc(&b.p, want) != hipSuccess) return {};
-    }
+    if (allocate(&b.p, want) != hipSuccess) return {};
     if (hipEventCreate(&b.clear_begin) != hipSuccess || hipEventCreate(&b.clear_end) != hipSuccess) {
         release(b);
         return {};
@@ -124,6 +158,15 @@ void CachePool::close() {
     drain();
 }
 
+namespace {
+
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return CachePool::allocate(reinterpret_cast<void**>(p), bytes);
+}
+
+}  // namespace
+
 // ------------------------------------------------------------------ Session
 Session::Session(Engine* engine, uint32_t capacity)
     : engine_(engine), capacity_(capacity), stride_((std::max<uint32_t>(capacity, 16) + 15) / 16 * 16) {
@@ -165,7 +208,7 @@ void Session::rollback(uint32_t n) {
 // ------------------------------------------------------------------ Engine
 void* Engine::device_alloc(size_t bytes) {
     void* p = nullptr;
-    if (hipMalloc(&p, bytes == 0 ? 16 : bytes) != hipSuccess) {
+    if (device_malloc(&p, bytes == 0 ? 16 : bytes) != hipSuccess) {
         fail(Status::OutOfMemory, "device allocation of " + std::to_string(bytes) + " bytes failed");
     }
     allocations_.push_back(p);
@@ -583,16 +626,13 @@ void Engine::ensure_capacity(uint32_t capacity) {
         if (*p) (void) hipFree(*p);
         *p = nullptr;
     }
-    hip_check(hipMalloc(&rope_, table.size() * sizeof(float)), "allocate rope table");
+    hip_check(device_malloc(&rope_, table.size() * sizeof(float)), "allocate rope table");
     hip_check(hipMemcpy(rope_, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice), "upload rope table");
     splits_ = gpu::attention_splits(static_cast<int32_t>(cap));
     attn_capacity_ = static_cast<int32_t>(cap);
     const size_t partial_floats = gpu::attention_partial_floats(gpu::kMaxRows, static_cast<int32_t>(p.n_head),
                                                                 static_cast<int32_t>(p.head_dim), splits_);
-    if (hipMalloc(&partial_, partial_floats * sizeof(float)) != hipSuccess) {
-        pool_->drain();
-        hip_check(hipMalloc(&partial_, partial_floats * sizeof(float)), "allocate attention partials");
-    }
+    hip_check(device_malloc(&partial_, partial_floats * sizeof(float)), "allocate attention partials");
     capacity_max_ = cap;
 }
 
@@ -1254,7 +1294,7 @@ void Engine::dequantize(const std::string& name, uint32_t row0, uint32_t n_rows,
     }
     float* dev = nullptr;
     const size_t bytes = static_cast<size_t>(n_rows) * m.cols * sizeof(float);
-    hip_check(hipMalloc(&dev, bytes), "allocate dequant output");
+    hip_check(device_malloc(&dev, bytes), "allocate dequant output");
     try {
         for (uint32_t i = 0; i < n_rows; ++i) {
             gpu::launch_dequant_rows(m, static_cast<int32_t>(device_row(ref, row0 + i)), 1,
@@ -1334,8 +1374,8 @@ void Engine::matmul(const std::string& name, const float* x_host, uint32_t n_tok
     const size_t x_bytes = static_cast<size_t>(n_tok) * m.cols * sizeof(float);
     const size_t y_bytes = static_cast<size_t>(n_tok) * m.rows * sizeof(float);
     float *x = nullptr, *y = nullptr;
-    hip_check(hipMalloc(&x, x_bytes), "allocate matmul input");
-    if (hipMalloc(&y, y_bytes) != hipSuccess) {
+    hip_check(device_malloc(&x, x_bytes), "allocate matmul input");
+    if (device_malloc(&y, y_bytes) != hipSuccess) {
         (void) hipFree(x);
         fail(Status::OutOfMemory, "allocate matmul output");
     }
@@ -1351,7 +1391,7 @@ void Engine::matmul(const std::string& name, const float* x_host, uint32_t n_tok
         gpu::Act8 xq;
         const int32_t blk = gpu::act_block(m.type);
         if (matmul_staged(m, n_tok)) {
-            hip_check(hipMalloc(&xq_mem, act8_bytes(n_tok, m.cols, blk)), "allocate int8 rows");
+            hip_check(device_malloc(&xq_mem, act8_bytes(n_tok, m.cols, blk)), "allocate int8 rows");
             xq = act8_at(xq_mem, n_tok, m.cols, blk);
         }
         run_matmul(m, x, n_tok, y, xq);

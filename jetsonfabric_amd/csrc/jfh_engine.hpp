@@ -59,8 +59,9 @@ struct BufferMetrics {
 };
 
 // Cache buffers of closed sessions, kept for the next ones: allocating and freeing device memory took longer than a
-// short prompt's first layers (7B, 100 rows: about 150 of 980 us per request). At most kBytes in kBuffers buffers,
-// given back with the engine and whenever an allocation fails. Sessions share it, since one may outlive its engine
+// short prompt's first layers (7B, 100 rows: about 150 of 980 us per request). At most kBytes in kBuffers buffers (a
+// 7B session of up to 4600 positions, a 32B one of up to 1000; longer ones are freed when they close), given back with
+// the engine and before any engine's allocation is refused. Sessions share it, since one may outlive its engine
 // and may be closed on any thread. Every step has finished when it returns, so a closed session's buffer is idle.
 class CachePool {
 public:
@@ -71,7 +72,10 @@ public:
         size_t size = 0;
         hipEvent_t clear_begin = nullptr, clear_end = nullptr;  // around its last clearing
     };
-    ~CachePool() { close(); }
+    CachePool();
+    ~CachePool();
+    // hipMalloc, once more without any engine's kept buffers if the memory does not suffice.
+    static hipError_t allocate(void** p, size_t bytes);
     // A buffer of at least `bytes`, p == nullptr when the device has no memory left.
     Buffer take(size_t bytes);
     void put(const Buffer& b);

@@ -103,10 +103,33 @@ void test_failed_capacity() {
     }
 }
 
+// Buffers kept for later sessions are given back before any allocation of any engine is refused.
+void test_kept_buffers_given_back() {
+    const auto e = engine();
+    { const auto warm = e->create_session(kCtx); }  // the rope table and partials of the longest session
+    const auto other = engine();
+    auto full = [&](auto&& call, const std::string& what) {
+        { const auto s = e->create_session(kCtx); }  // 8 MB, kept
+        fake::memory = fake::live_bytes;
+        try {
+            call();
+        } catch (const Error& err) {
+            expect(false, what + ": " + err.what());
+        }
+        fake::memory = ~size_t{0};
+    };
+    std::vector<float> x(kEmbd), y(kVocab * kEmbd);
+    full([&] { e->matmul("blk.0.attn_output.weight", x.data(), 1, y.data()); }, "matmul");
+    full([&] { e->dequantize("blk.0.attn_output.weight", 0, 1, y.data()); }, "dequantize");
+    full([&] { (void) other->create_session(1000); }, "another engine's session");
+    full([&] { (void) other->create_session(1050); }, "another engine's rope table and partials");
+}
+
 }  // namespace
 
 int main() {
     test_failed_capacity();
+    test_kept_buffers_given_back();
     test_allocation_time();
     test_prefill_scratch();
     failures += fake::faults;

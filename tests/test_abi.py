@@ -84,6 +84,15 @@ def test_matmul_route_cpp_tests():
     assert "route tests passed" in r.stdout
 
 
+def test_engine_on_host_memory_cpp_tests():
+    """The engine on a device in host memory: prefill figures and chunks, session buffers, refused allocations."""
+    exe = os.path.join(ROOT, "tests", "cpp", "engine_test")
+    subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "cpp")], check=True, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "engine tests passed" in r.stdout
+
+
 def test_engine_creation_fails_loudly_without_a_gpu():
     import torch
 
