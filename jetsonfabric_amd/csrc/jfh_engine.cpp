@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <thread>
 
 namespace jfh {
 namespace {
@@ -174,6 +175,7 @@ Session::Session(Engine* engine, uint32_t capacity)
     const size_t elems = static_cast<size_t>(engine->resident_layers()) * p.n_head_kv * stride_ * p.head_dim;
     kv_bytes_ = 2 * elems * sizeof(uint16_t);
     pool_ = engine->pool_;
+    activity_ = engine->activity_;
     buffer_ = pool_->take(kv_bytes_);
     if (buffer_.p == nullptr) fail(Status::OutOfMemory, "allocate K and V cache");
     k_ = static_cast<uint16_t*>(buffer_.p);
@@ -188,7 +190,11 @@ Session::Session(Engine* engine, uint32_t capacity)
     }
 }
 
-Session::~Session() { pool_->put(buffer_); }
+Session::~Session() {
+    const Session* self = this;
+    activity_->session.compare_exchange_strong(self, nullptr);
+    pool_->put(buffer_);
+}
 
 double Session::clear_ms() const {
     float ms = 0.0F;
@@ -640,7 +646,7 @@ std::unique_ptr<Session> Engine::create_session(uint32_t capacity) {
     if (capacity == 0 || capacity > params_.n_ctx) {
         fail(Status::InvalidArgument, "native Qwen2 cache capacity is outside model context");
     }
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     ensure_capacity(capacity);
     const auto t0 = std::chrono::steady_clock::now();
     std::unique_ptr<Session> s(new Session(this, capacity));
@@ -863,7 +869,7 @@ void Engine::record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_ou
 }
 
 void Engine::read_kv(const Session& s, uint32_t layer, uint32_t n, uint16_t* k, uint16_t* v) {
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     const ModelParams& p = params_;
     if (layer < layer_start_ || layer >= layer_end_ || n > s.position_) {
         fail(Status::InvalidArgument, "cache rows are outside the session");
@@ -885,7 +891,7 @@ void Engine::read_kv(const Session& s, uint32_t layer, uint32_t n, uint16_t* k, 
 }
 
 void Engine::import_kv(Session& s, uint32_t n, const uint16_t* k, const uint16_t* v) {
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     const ModelParams& p = params_;
     if (n == 0 || n > s.capacity_) fail(Status::InvalidArgument, "imported cache rows exceed the session capacity");
     hip_check(hipStreamSynchronize(stream_), "synchronize before cache import");
@@ -924,7 +930,7 @@ std::vector<KernelStat> Engine::profile(const std::vector<SeqStep>& steps, uint3
         std::vector<int32_t> ids(gpu::kMaxRows);
         for (uint32_t it = 0; it < iterations; ++it) {
             // a single sequence's step may be a whole prefill chunk
-            forward(steps, ids.data(), nullptr, nullptr, nullptr, nullptr,
+            forward(steps, ids.data(), nullptr, nullptr, nullptr,
                     steps.size() == 1 ? std::max<uint32_t>(gpu::kMaxRows, prefill_chunk_) : gpu::kMaxRows);
             for (const SeqStep& st : steps) st.session->position_ -= st.n;
         }
@@ -994,11 +1000,33 @@ std::vector<int32_t> Engine::end_tokens() const {
     return end_tokens_;
 }
 
+void Engine::Queue::let_pass() const {
+    for (const uint64_t until = turns + waiting; waiting > 0 && turns < until;) {
+        std::this_thread::sleep_for(std::chrono::microseconds(10));
+    }
+}
+
+Engine::Turn::Turn(Engine& e, Kind kind) : e_(e) {
+    Queue& own = kind == kStep ? e.steps_ : e.others_;
+    (kind == kStep ? e.others_ : e.steps_).let_pass();
+    own.waiting.fetch_add(1);
+    e.mutex_.lock();
+    own.turns.fetch_add(1);
+    own.waiting.fetch_sub(1);
+}
+
 void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits,
-                     float* act_out, PrefillMetrics* metrics, uint32_t row_limit) {
+                     float* act_out, uint32_t row_limit) {
+    Turn turn(*this, Turn::kStep);
+    run(steps, out_tokens, accepted, logits, act_out, nullptr, row_limit, 0);
+    activity_->session = steps.back().session;
+    activity_->at_ns = std::chrono::steady_clock::now().time_since_epoch().count();
+}
+
+void Engine::run(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits,
+                 float* act_out, PrefillMetrics* metrics, uint32_t row_limit, uint32_t prompt) {
     using clock = std::chrono::steady_clock;
     const auto ms_since = [](clock::time_point t) { return std::chrono::duration<double, std::milli>(clock::now() - t).count(); };
-    std::lock_guard lock(mutex_);
     const auto t_input = clock::now();
     const ModelParams& p = params_;
     if (!last_stage() && act_out == nullptr) fail(Status::InvalidArgument, "a non-final stage needs an activation output");
@@ -1090,11 +1118,13 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
         metrics->attention_matrix_cores = p.head_dim == 64 || p.head_dim == 128;
         ++metrics->steps;
     }
-    const bool whole_keys = gpu::attention_prefill_supported(
+    // Every chunk of a prompt longer than a step runs the attention that does not depend on where the prompt is cut, and
+    // without a graph: its kernels outlast their launches, and its row count is not met again.
+    const bool cut_prompt = prompt > static_cast<uint32_t>(gpu::kMaxRows) && prefill_chunk_ > static_cast<uint32_t>(gpu::kMaxRows);
+    const bool whole_keys = cut_prompt || gpu::attention_prefill_supported(
         rows, sd.n_seq, static_cast<int32_t>(p.n_head), static_cast<int32_t>(p.n_head_kv), static_cast<int32_t>(p.head_dim),
         sd.seqs[0].pos0 + sd.seqs[0].len);
-    // a long chunk's kernels outlast their launches: no graph is captured for its row count
-    if (options_.use_graphs && rows <= gpu::kMaxRows) {
+    if (options_.use_graphs && rows <= gpu::kMaxRows && !cut_prompt) {
         const uint64_t key = (whole_keys ? uint64_t{1} << 63 : 0) | (static_cast<uint64_t>(rows) << 40) | (static_cast<uint64_t>(max_len) << 32) |
                              (static_cast<uint64_t>(steps.size()) << 16) | (static_cast<uint64_t>(outs) << 1) |
                              (store ? 1u : 0u);
@@ -1194,24 +1224,41 @@ uint32_t Engine::balanced_chunk(uint32_t n) const {
     return std::min(prefill_chunk_, ((n + chunks - 1) / chunks + 127) / 128 * 128);
 }
 
-int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* logits) {
-    require_full_model();
-    if (s.position_ != 0 || n == 0 || n > s.capacity_) {
-        fail(Status::InvalidArgument, "native Qwen2 prefill is outside session capacity");
-    }
+// Rows of a prompt's next chunk, `left` being left. A chunk holds the engine until it has run, for 14B and 2048 rows
+// about 100 ms; while another session steps, chunks are kBusyChunk rows long, which hold it no longer than the 256-row
+// chunks of the split-key attention did (one layer at 4096 positions, 384 rows now and 256 then: 14B Q4_K 521 and
+// 599 us, 7B Q4_K 486 and 474, 32B Q2_K 717 and 1943; models of few heads longer, 1.5B 279 and 185). Another session
+// steps if one waits now or an open one stepped within kBusyNs, several times what a decode loop spends between steps.
+uint32_t Engine::next_chunk(uint32_t left, bool steps_between) {
+    constexpr uint32_t kBusyChunk = 384;
+    constexpr int64_t kBusyNs = 20'000'000;
+    const bool busy = steps_.waiting > 0 ||
+                      (steps_between && activity_->session != nullptr &&
+                       std::chrono::steady_clock::now().time_since_epoch().count() - activity_->at_ns < kBusyNs);
+    const uint32_t chunk = balanced_chunk(left);
+    return std::min(left, busy ? std::min(chunk, kBusyChunk) : chunk);
+}
+
+int32_t Engine::run_prompt(Session& s, const int32_t* tokens, const float* activations, uint32_t n, float* act_out,
+                           float* logits, bool steps_between) {
+    const size_t H = params_.n_embd;
     int32_t token = -1;
     PrefillMetrics m;
     m.allocation_ms = s.prefill_metrics_.allocation_ms;
-    const uint32_t chunk = balanced_chunk(n);
     for (uint32_t done = 0; done < n;) {
-        const uint32_t len = std::min(chunk, n - done);
+        const uint32_t len = next_chunk(n - done, steps_between);
         const bool last = done + len == n;
         SeqStep st;
         st.session = &s;
-        st.tokens = tokens + done;
+        st.tokens = tokens ? tokens + done : nullptr;
+        st.activations = activations ? activations + done * H : nullptr;
         st.n = len;
-        st.logits = last ? 1 : 0;
-        forward({st}, last ? &token : nullptr, nullptr, last ? logits : nullptr, nullptr, &m, prefill_chunk_);
+        st.logits = last && last_stage() ? 1 : 0;
+        {
+            Turn turn(*this, Turn::kOther);
+            run({st}, st.logits ? &token : nullptr, nullptr, st.logits ? logits : nullptr,
+                act_out ? act_out + done * H : nullptr, &m, prefill_chunk_, n);
+        }
         done += len;
     }
     s.prefill_position_ = n;
@@ -1221,8 +1268,16 @@ int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* lo
     return token;
 }
 
+int32_t Engine::prefill(Session& s, const int32_t* tokens, uint32_t n, float* logits, bool steps_between) {
+    require_full_model();
+    if (s.position_ != 0 || n == 0 || n > s.capacity_) {
+        fail(Status::InvalidArgument, "native Qwen2 prefill is outside session capacity");
+    }
+    return run_prompt(s, tokens, nullptr, n, nullptr, logits, steps_between);
+}
+
 int32_t Engine::stage_prefill(Session& s, const int32_t* tokens, const float* activations, uint32_t n,
-                              float* act_out, float* logits) {
+                              float* act_out, float* logits, bool steps_between) {
     if (first_stage() && activations != nullptr) {
         fail(Status::InvalidArgument, "the first native stage does not accept activations");
     }
@@ -1235,29 +1290,7 @@ int32_t Engine::stage_prefill(Session& s, const int32_t* tokens, const float* ac
     if (s.position_ != 0 || n == 0 || n > s.capacity_) {
         fail(Status::InvalidArgument, "native Qwen2 prefill is outside session capacity");
     }
-    const size_t H = params_.n_embd;
-    int32_t token = -1;
-    PrefillMetrics m;
-    m.allocation_ms = s.prefill_metrics_.allocation_ms;
-    const uint32_t chunk = balanced_chunk(n);
-    for (uint32_t done = 0; done < n;) {
-        const uint32_t len = std::min(chunk, n - done);
-        const bool last = done + len == n;
-        SeqStep st;
-        st.session = &s;
-        st.tokens = tokens ? tokens + done : nullptr;
-        st.activations = activations ? activations + done * H : nullptr;
-        st.n = len;
-        st.logits = last && last_stage() ? 1 : 0;
-        forward({st}, st.logits ? &token : nullptr, nullptr, st.logits ? logits : nullptr,
-                act_out ? act_out + done * H : nullptr, &m, prefill_chunk_);
-        done += len;
-    }
-    s.prefill_position_ = n;
-    m.allocation_ms += s.clear_ms();
-    s.prefill_metrics_ = m;
-    t_last_prefill = m;
-    return token;
+    return run_prompt(s, tokens, activations, n, act_out, logits, steps_between);
 }
 
 int32_t Engine::stage_decode(Session& s, const int32_t* token, const float* activation, float* act_out,
@@ -1286,7 +1319,7 @@ int32_t Engine::stage_decode(Session& s, const int32_t* token, const float* acti
 }
 
 void Engine::dequantize(const std::string& name, uint32_t row0, uint32_t n_rows, float* out_host) {
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     const TensorRef& ref = find_ref(name);
     const gpu::DMat& m = ref.dev->mat;
     if (n_rows == 0 || static_cast<uint64_t>(row0) + n_rows > ref.rows) {
@@ -1364,7 +1397,7 @@ void Engine::run_matmul(const gpu::DMat& m, const float* x, uint32_t n_tok, floa
 }
 
 void Engine::matmul(const std::string& name, const float* x_host, uint32_t n_tok, float* y_host) {
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     const TensorRef& ref = find_ref(name);
     const gpu::DMat& m = ref.dev->mat;
     if (n_tok == 0 || n_tok > static_cast<uint32_t>(gpu::kMaxRows)) {
@@ -1411,7 +1444,7 @@ void Engine::matmul(const std::string& name, const float* x_host, uint32_t n_tok
 
 void Engine::matmul_noalloc(const std::string& name, const float* x_dev, uint32_t n_tok, float* y_dev,
                             hipStream_t after) {
-    std::lock_guard lock(mutex_);
+    Turn turn(*this, Turn::kOther);
     const TensorRef& ref = find_ref(name);
     const gpu::DMat& m = ref.dev->mat;
     if (n_tok == 0 || n_tok > static_cast<uint32_t>(gpu::kMaxRows)) {

@@ -12,6 +12,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -30,6 +31,7 @@ struct EngineOptions {
 };
 
 class Engine;
+class Session;
 
 // KV-cache owner; position bookkeeping follows Qwen2Session
 // (qwen2_architecture.cpp:800-823, 1040-1054).
@@ -90,6 +92,13 @@ private:
     bool closed_ = false;
 };
 
+// The session that stepped last and when (steady_clock ns): whether a prefill shares the engine. Kept by the engine and
+// its sessions, since one may be closed on any thread or outlive its engine.
+struct StepActivity {
+    std::atomic<const Session*> session{nullptr};
+    std::atomic<int64_t> at_ns{0};
+};
+
 class Session {
 public:
     ~Session();
@@ -116,6 +125,7 @@ private:
     uint32_t position_ = 0;
     uint32_t prefill_position_ = 0;
     std::shared_ptr<CachePool> pool_;
+    std::shared_ptr<StepActivity> activity_;
     CachePool::Buffer buffer_;  // holds K, then V
     uint16_t* k_ = nullptr;  // [resident layer][kv head][stride][head_dim]
     uint16_t* v_ = nullptr;  // [resident layer][kv head][stride / 16][head_dim][16] (16-position tiles)
@@ -179,15 +189,17 @@ public:
     // sequence; logits (optional) n_logits_rows x vocab floats. A stage
     // that is not the last one computes no logits: act_out receives the
     // residual-stream rows after its last layer, f32 [rows][n_embd].
-    // metrics (optional) accumulates the step's host and device times. A step has
-    // at most row_limit rows (a prefill chunk of one sequence up to
-    // max_prefill_chunk).
+    // A step has at most row_limit rows.
     void forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits,
-                 float* act_out = nullptr, PrefillMetrics* metrics = nullptr, uint32_t row_limit = gpu::kMaxRows);
+                 float* act_out = nullptr, uint32_t row_limit = gpu::kMaxRows);
 
     // Prefill of arbitrary length: runs the prompt in chunks and returns the
-    // greedy token of the last row (and its logits if requested).
-    int32_t prefill(Session& s, const int32_t* tokens, uint32_t n, float* logits);
+    // greedy token of the last row (and its logits if requested). Steps that
+    // other threads run meanwhile take turns with the chunks (next_chunk); the
+    // results do not depend on how the prompt is cut. A caller that lets no
+    // other session step before the prefill has returned says so with
+    // steps_between = false.
+    int32_t prefill(Session& s, const int32_t* tokens, uint32_t n, float* logits, bool steps_between = true);
 
     // One pipeline stage's prefill (n rows at position 0) or decode (one row)
     // (Qwen2Session::prefill_stage_* / decode_stage_*,
@@ -197,7 +209,7 @@ public:
     // act_out and return -1. The last stage also writes the last row's
     // logits to `logits` when it is set.
     int32_t stage_prefill(Session& s, const int32_t* tokens, const float* activations, uint32_t n, float* act_out,
-                          float* logits = nullptr);
+                          float* logits = nullptr, bool steps_between = true);
     int32_t stage_decode(Session& s, const int32_t* token, const float* activation, float* act_out,
                          float* logits = nullptr);
 
@@ -268,7 +280,32 @@ private:
     const TensorRef& find_ref(const std::string& name) const;
     const float* upload_f32(const TensorView& t);
     void ensure_capacity(uint32_t capacity);
+    // Steps, or the other calls (prefill chunks, session calls), that wait for the engine's lock and that have had it.
+    // The lock itself favours the thread that has just released it, so the chunks of a prefill would run one after
+    // another, and the steps of a decode loop: each kind lets the other's waiting ones go first.
+    struct Queue {
+        std::atomic<uint32_t> waiting{0};
+        std::atomic<uint64_t> turns{0};
+        void let_pass() const;
+    };
+    class Turn {
+    public:
+        enum Kind { kStep, kOther };
+        Turn(Engine& e, Kind kind);
+        ~Turn() { e_.mutex_.unlock(); }
+        Turn(const Turn&) = delete;
+        Turn& operator=(const Turn&) = delete;
+
+    private:
+        Engine& e_;
+    };
     uint32_t balanced_chunk(uint32_t n) const;
+    uint32_t next_chunk(uint32_t left, bool steps_between);
+    // One step, or with prompt > 0 one chunk of a prompt of that many rows; the caller holds the lock.
+    void run(const std::vector<SeqStep>& steps, int32_t* out_tokens, int32_t* accepted, float* logits, float* act_out,
+             PrefillMetrics* metrics, uint32_t row_limit, uint32_t prompt);
+    int32_t run_prompt(Session& s, const int32_t* tokens, const float* activations, uint32_t n, float* act_out,
+                       float* logits, bool steps_between);
     void record(int32_t n_rows, int32_t max_len, int32_t n_seq, int32_t n_out, bool store_logits, bool whole_keys);
     template <typename F>
     void timed(const std::string& label, double bytes, F&& fn);
@@ -328,6 +365,8 @@ private:
     std::map<uint64_t, hipGraphExec_t> graphs_;
     std::vector<int32_t> end_tokens_;
     mutable std::mutex mutex_;
+    Queue steps_, others_;
+    std::shared_ptr<StepActivity> activity_ = std::make_shared<StepActivity>();
 };
 
 }  // namespace jfh

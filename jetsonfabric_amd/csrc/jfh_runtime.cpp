@@ -657,7 +657,7 @@ private:
         std::vector<float> out_rows(config.position.is_last() ? 0 : count * config.engine->params().n_embd);
         const std::int32_t token = config.engine->stage_prefill(
             *session, tokens.empty() ? nullptr : tokens.data(), act.empty() ? nullptr : act.data(),
-            static_cast<std::uint32_t>(count), out_rows.empty() ? nullptr : out_rows.data());
+            static_cast<std::uint32_t>(count), out_rows.empty() ? nullptr : out_rows.data(), nullptr, false);
         StageOutput out = config.position.is_last() ? token_output(token) : activation_output(out_rows);
         if (config.position.is_first()) {
             out.prompt_tokens = static_cast<int>(tokens.size());
@@ -705,7 +705,8 @@ private:
         const std::size_t capacity = session_capacity(tokens.size(), in.max_tokens);
         std::unique_ptr<Session> session = config.engine->create_session(static_cast<std::uint32_t>(capacity));
         const std::int32_t token =
-            config.engine->prefill(*session, tokens.data(), static_cast<std::uint32_t>(tokens.size()), nullptr);
+            // this executor's lock is held: none of its sessions steps meanwhile
+            config.engine->prefill(*session, tokens.data(), static_cast<std::uint32_t>(tokens.size()), nullptr, false);
         StageOutput out = token_output(token);
         out.prompt_tokens = static_cast<int>(tokens.size());
         for (const std::int32_t t : tokens) {

@@ -29,6 +29,7 @@ inline double clock_ms = 0.0;
 inline int faults = 0;                    // copies, fills and frees outside an allocation
 inline int captures = 0;
 inline std::atomic<uint32_t> step_rows{0};      // rows of the step being launched
+inline std::atomic<uint32_t> longest_step{0};
 inline std::atomic<int> us_per_256_rows{0};     // real time a step's synchronization takes
 
 inline void fault(const char* what) {
@@ -131,6 +132,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = reinterpret
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) {
     const uint32_t rows = fake::step_rows.exchange(0);
+    if (rows > fake::longest_step) fake::longest_step = rows;
     if (rows > 0) std::this_thread::sleep_for(std::chrono::microseconds(fake::us_per_256_rows * ((rows + 255) / 256)));
     return hipSuccess;
 }

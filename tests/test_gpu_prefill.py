@@ -1,4 +1,7 @@
 """Long steps: the prefill matmul tiles and the attention of whole prefill chunks."""
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -101,3 +104,51 @@ def test_reused_cache_buffers_start_clean():
     used.close()
     late.close()
     fresh.close()
+
+
+# 8 heads x 64 and 5 x 128; 385 and 769 rows leave a last chunk of one row when cut, 2200 is cut in any case.
+@pytest.mark.parametrize("n_head,n_head_kv,head_dim", [(8, 2, 64), (10, 2, 128)])
+@pytest.mark.parametrize("n", [385, 769, 1000, 2200])
+def test_prompt_cut_for_other_sessions_is_the_same(n_head, n_head_kv, head_dim, n):
+    """A prompt run in short chunks because another session steps gives the logits and the cache of the same prompt run
+    alone, bit for bit, also while that session goes on stepping on another thread; so do its steps."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=n_head * head_dim, n_ff=768, n_head=n_head, n_head_kv=n_head_kv, n_vocab=512,
+                         n_ctx=4096)
+    engine = jf.NativeEngine(jf.Model.synthesize(cfg, type_linear=jf.Q4_K, type_embd=jf.Q4_K, type_output=jf.Q6_K, seed=n))
+    try:
+        tokens = [int(t) for t in np.random.default_rng(n).integers(0, cfg.n_vocab, n)]
+
+        def prefill():
+            s = engine.create_session(n + 8)
+            logits = s.prefill_greedy(tokens, logits=True)[1]
+            k, v = s.read_kv(1, n)
+            s.close()
+            return logits.view(np.uint32), np.asarray(k), np.asarray(v)
+
+        def greedy(s, count, stop=lambda: False):
+            ids = [s.prefill_greedy(tokens[:30])]
+            while len(ids) < count and not stop():
+                ids.append(s.decode_greedy(ids[-1]))
+            return ids
+
+        alone = prefill()
+        s = engine.create_session(4000)
+        expected = greedy(s, 60)
+        assert all(np.array_equal(a, b) for a, b in zip(alone, prefill()))  # it has just stepped
+        s.close()
+
+        s, done, got = engine.create_session(4000), threading.Event(), []
+        decoder = threading.Thread(target=lambda: got.extend(greedy(s, 3900, done.is_set)))
+        decoder.start()
+        try:
+            while s.position() < 32:
+                time.sleep(1e-4)
+            for _ in range(3):
+                assert all(np.array_equal(a, b) for a, b in zip(alone, prefill()))
+        finally:
+            done.set()
+            decoder.join()
+        assert len(got) > 4 and got[:60] == expected[:len(got)]
+        s.close()
+    finally:
+        engine.close()
