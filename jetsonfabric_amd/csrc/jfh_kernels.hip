@@ -2094,7 +2094,7 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_wide(GemvArgs a, int32_t n_rg
 constexpr int kStageRow = 272;  // bytes per staged token row: 256 codes + 16 bytes of padding (banks)
 
 template <int NW, int TP>
-__global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t n_rg, int32_t tpw) {
+__global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t n_rg) {
     constexpr int NTHR = NW * kWave;
     constexpr int NTOK = 16 * TP;
     constexpr uint32_t TB = tile_bytes(11);
@@ -2108,19 +2108,13 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
     __shared__ float scales[2][NTOK];
     static_assert(sizeof(float) * NTOK * VSTRIDE <= sizeof(codes), "epilogue values alias the staging buffers");
     float* vals = reinterpret_cast<float*>(&codes[0][0]);
-    const int n_tok = a.n_tok, n_tt = (n_tok + 15) / 16, n_grp = (n_tt + tpw - 1) / tpw;
-    const int n_sets = (n_rg + NW - 1) / NW;
-    // work-group k runs on XCD k % 8: the token groups of one row-group set share an XCD (and its L2)
-    const int q = static_cast<int>(blockIdx.x) >> 3;
-    const int grp = q % n_grp, set = (q / n_grp) * 8 + static_cast<int>(blockIdx.x & 7u);
-    if (set >= n_sets) return;
+    const int n_tok = a.n_tok;  // 16 (TP - 1) + 1 .. 16 TP
+    const int set = static_cast<int>(blockIdx.x);
+    if (set * NW >= n_rg) return;
     const int K = static_cast<int>(a.mat.cols), nb = K / 256;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
     const int i = lane & 15, G = lane >> 4;
-    const int tt0 = grp * tpw, ntl = min(TP, min(n_tt, tt0 + tpw) - tt0);
-    const int t0 = 16 * tt0, nt = min(16 * (tt0 + ntl), n_tok) - t0;
-    const GemvArgs out = token_slice(a, t0, nt);
     const Act8 xq = a.xq;
     const int rg = set * NW + wave;
     const bool active = rg < n_rg;  // waves past the matrix stage and wait but compute nothing
@@ -2138,15 +2132,15 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
 #pragma unroll
         for (int u = 0; u < CPT; ++u) {
             const uint32_t e = threadIdx.x + u * NTHR, tk = e >> 4, part = e & 15;
-            const uint32_t tok = static_cast<uint32_t>(min(t0 + static_cast<int>(tk), n_tok - 1));
+            const uint32_t tok = static_cast<uint32_t>(min(static_cast<int>(tk), n_tok - 1));
             st.c[u] = *reinterpret_cast<const u32x4*>(xq.q + (tok * static_cast<uint32_t>(K) + 256u * b + 16u * part));
         }
         if (threadIdx.x < 2 * NTOK) {
-            const uint32_t tok = static_cast<uint32_t>(min(t0 + static_cast<int>(threadIdx.x >> 1), n_tok - 1));
+            const uint32_t tok = static_cast<uint32_t>(min(static_cast<int>(threadIdx.x >> 1), n_tok - 1));
             st.s = *reinterpret_cast<const u32x4*>(xq.s + (tok * static_cast<uint32_t>(K / 16) + 16u * b + 8u * (threadIdx.x & 1)));
         }
         if (threadIdx.x < NTOK) {
-            const uint32_t tok = static_cast<uint32_t>(min(t0 + static_cast<int>(threadIdx.x), n_tok - 1));
+            const uint32_t tok = static_cast<uint32_t>(min(static_cast<int>(threadIdx.x), n_tok - 1));
             st.d = xq.d[tok * static_cast<uint32_t>(nb) + b];
         }
         return st;
@@ -2235,26 +2229,24 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
             }
 #pragma unroll
             for (int tl = 0; tl < TP; ++tl) {
-                if (tl < ntl) {
-                    const int r = 16 * tl + i;
-                    const u32x4* src = reinterpret_cast<const u32x4*>(&codes[buf][r * kStageRow + 64 * G]);
-                    const float2 xs = reinterpret_cast<const float2*>(&sums[buf][r][0])[G];
-                    const float xd = scales[buf][r];
-                    i32x4 DL = {0, 0, 0, 0}, DH = {0, 0, 0, 0};
+                const int r = 16 * tl + i;
+                const u32x4* src = reinterpret_cast<const u32x4*>(&codes[buf][r * kStageRow + 64 * G]);
+                const float2 xs = reinterpret_cast<const float2*>(&sums[buf][r][0])[G];
+                const float xd = scales[buf][r];
+                i32x4 DL = {0, 0, 0, 0}, DH = {0, 0, 0, 0};
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) {
-                        const i32x4 av = __builtin_bit_cast(i32x4, src[m]);
-                        DL = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, BL[m]), av, DL, 0, 0, 0);
-                        DH = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, BH[m]), av, DH, 0, 0, 0);
-                    }
-                    // token r's 32-value code sums of sub-blocks 2G, 2G + 1
-                    f32x4 ms = {0.0F, 0.0F, 0.0F, 0.0F};
-                    ms = __builtin_amdgcn_mfma_f32_16x16x4f32(ma, xs.x, ms, 0, 0, 0);
-                    ms = __builtin_amdgcn_mfma_f32_16x16x4f32(mb, xs.y, ms, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        chain[tl][j] = q4k_term_f(chain[tl][j], xd, d[j], dmin[j], DL[j] + 8 * DH[j], ms[j]);
+                for (int m = 0; m < 4; ++m) {
+                    const i32x4 av = __builtin_bit_cast(i32x4, src[m]);
+                    DL = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, BL[m]), av, DL, 0, 0, 0);
+                    DH = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, BH[m]), av, DH, 0, 0, 0);
                 }
+                // token r's 32-value code sums of sub-blocks 2G, 2G + 1
+                f32x4 ms = {0.0F, 0.0F, 0.0F, 0.0F};
+                ms = __builtin_amdgcn_mfma_f32_16x16x4f32(ma, xs.x, ms, 0, 0, 0);
+                ms = __builtin_amdgcn_mfma_f32_16x16x4f32(mb, xs.y, ms, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    chain[tl][j] = q4k_term_f(chain[tl][j], xd, d[j], dmin[j], DL[j] + 8 * DH[j], ms[j]);
             }
             if (b + 8 >= nb) {
                 // the chain of tiles b mod 8 ends: its partial joins the total in wave order
@@ -2284,7 +2276,7 @@ __global__ __launch_bounds__(NW * kWave) void k_mm_wide_q4k(GemvArgs a, int32_t 
     __syncthreads();
     const int row0 = set * NW * 16;
     const int nrows = min(16 * NW, static_cast<int>(a.mat.rows) - row0);
-    gemv_epilogue<NTHR, kNoLogits>(out, row0, nrows, [&](int j, int tk) { return vals[tk * VSTRIDE + j]; }, nullptr);
+    gemv_epilogue<NTHR, kNoLogits>(a, row0, nrows, [&](int j, int tk) { return vals[tk * VSTRIDE + j]; }, nullptr);
 }
 
 // ------------------------------------------------------------------ long-step matmul
@@ -4276,9 +4268,9 @@ void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
         const MmRoute r = mm_route(a.mat.type, a.mat.rows, a.mat.cols, a.n_tok);
         if (r.kernel != MmKernel::kWide) {
             if (r.kernel == MmKernel::kStream) {
-                const dim3 g(((n_rg + kWideQ4kWaves - 1) / kWideQ4kWaves + 7) / 8 * 8), b(kWideQ4kWaves * kWave);
-                if (r.tiles == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg, 2);
-                else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg, 1);
+                const dim3 g((n_rg + kWideQ4kWaves - 1) / kWideQ4kWaves), b(kWideQ4kWaves * kWave);
+                if (r.tiles == 2) launch(k_mm_wide_q4k<kWideQ4kWaves, 2>, g, b, 0, stream, a, n_rg);
+                else launch(k_mm_wide_q4k<kWideQ4kWaves, 1>, g, b, 0, stream, a, n_rg);
             } else if (a.mat.type == 7) {
                 if (r.tiles == 2) gemm<7, 2, 3>(a, n_rg, n_tt, stream);
                 else gemm<7, 1, 4>(a, n_rg, n_tt, stream);
@@ -4300,18 +4292,10 @@ void launch_gemv_wide(const GemvArgs& a_in, hipStream_t stream) {
         if (merged) go(k_mm_wide<7, true, true>);
         else go(k_mm_wide<7, false, true>);
         break;
-    case 9:
-        if (merged) go(k_mm_wide<9, true, false>);
-        else go(k_mm_wide<9, false, false>);
-        break;
-    case 11:
-        if (merged) go(k_mm_wide<11, true, false>);
-        else go(k_mm_wide<11, false, false>);
-        break;
-    default:
-        if (merged) go(k_mm_wide<13, true, false>);
-        else go(k_mm_wide<13, false, false>);
-        break;
+    // the K-quants' layer matrices run on the folded tiles
+    case 9: go(k_mm_wide<9, true, false>); break;
+    case 11: go(k_mm_wide<11, true, false>); break;
+    default: go(k_mm_wide<13, true, false>); break;
     }
     check(hipGetLastError(), "wide matmul launch");
 }
