@@ -2501,10 +2501,13 @@ struct GemmTile<7> {
 
 // Copies 16 bytes per lane from base + off to LDS at lds + 16 * lane (lds is wave-uniform), past the
 // registers. The compiler does not count these loads: lds_dma_wait before the barrier that publishes them.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register: it is named so that no copy of it lives across
 __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
                  : "memory", "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // The epilogue of a whole 64-row set: the same values as gemv_epilogue's, four rows per thread and the set's tokens
