@@ -103,7 +103,7 @@ def test_failing_draft_strategy_proposes_nothing(engine):
 
 
 def test_generation_metrics(engine):
-    prompt = _prompt(300, 6)  # several prefill chunks
+    prompt = _prompt(300, 6)  # one prefill chunk, longer than a step
     n = 12
     first = engine.generate(prompt, n)
     again = engine.generate(prompt, n)
@@ -132,7 +132,16 @@ def test_generation_metrics(engine):
         row = (3 * CFG.n_embd + CFG.n_ff) * 4 + 2 * act8(CFG.n_embd) + act8(CFG.n_ff)
         assert b["decode_scratch_bytes"] > row + CFG.n_vocab * 4
         assert b["prefill_scratch_bytes"] == 300 * row + 256 * (b["decode_scratch_bytes"] - row)
-    # the second run replays the step graphs the first one captured
+    assert first.sampled_tokens == again.sampled_tokens
+    # beyond one step a prompt runs without graphs
+    assert first.prefill["plan_reused"] and first.prefill["planning_ms"] == 0.0
+
+
+def test_generation_captures_a_prompt_step_once(engine):
+    """The first prompt of a row count captures its step's graph, the second replays it."""
+    prompt = _prompt(211, 61)
+    first, again = engine.generate(prompt, 6), engine.generate(prompt, 6)
+    assert not first.prefill["plan_reused"] and first.prefill["planning_ms"] > 0.0
     assert again.prefill["plan_reused"] and again.prefill["planning_ms"] == 0.0
     assert first.sampled_tokens == again.sampled_tokens
 

@@ -151,9 +151,9 @@ def test_wide_matmul_over_row_group_sets_equals_single_rows(wide_typed):
 
 # A Q4_K gate/up matrix of 16384 rows (256 sets of four row groups) over K =
 # 2560 (ten tiles: the decode waves' chains of two and one tiles): steps of
-# 9..256 rows run the whole-K-wave kernel that folds the sub-block scales into
-# the weight operand and shares each activation tile through LDS (steps of more
-# than 64 rows as several token groups of four 16-token tiles).
+# 9..32 rows run the streaming kernel, longer ones the long-step kernel, both
+# with whole-K waves that fold the sub-block scales into the weight operand and
+# share each activation tile through LDS.
 WIDE_Q4 = jf.ModelConfig(n_layer=1, n_embd=2560, n_ff=8192, n_head=20, n_head_kv=4, n_vocab=4096, n_ctx=512)
 
 
@@ -186,8 +186,8 @@ def test_folded_scale_wide_matmul_equals_single_rows(wide_q4):
 
 
 def test_folded_scale_prefill_matches_oracle_and_token_by_token(wide_q4):
-    """A 300-token prompt (chunks of 256 and 44 rows: the SwiGLU gate/up
-    matrix on the folded-scale kernel) matches the oracle's logits, and a
+    """A 300-token prompt (one chunk: the SwiGLU gate/up matrix on the
+    long-step kernel) matches the oracle's logits, and a
     session fed the prompt one token at a time reaches the same greedy
     continuation."""
     model, engine, om = wide_q4
@@ -239,7 +239,7 @@ def test_forward_matches_oracle(q4k):
 
 
 def test_chunked_prefill_matches_oracle_and_token_by_token(q4k):
-    """A 300-token prompt is prefilled in chunks of up to 256 rows (matrix-core
+    """A 300-token prompt is prefilled in one chunk, longer than a step (matrix-core
     matmuls); its logits match the oracle's, and a session fed the same
     prompt one token at a time reaches the same greedy continuation."""
     model, engine, om = q4k

@@ -152,3 +152,90 @@ def test_prompt_cut_for_other_sessions_is_the_same(n_head, n_head_kv, head_dim, 
         s.close()
     finally:
         engine.close()
+
+
+# The two-row-group form of the chunk attention (grids of 512 work-groups of 128 query rows or more): a ragged chunk of
+# 1900 rows and, after a chunk of 1152, one of 1000. Head dims 128 and 64, one head per kv head.
+@pytest.mark.parametrize("n_head,n_head_kv,head_dim,n", [(40, 8, 128, 1900), (40, 8, 64, 1900), (64, 16, 64, 2152), (36, 36, 64, 1900)])
+def test_wide_chunk_attention_matches_short_steps(n_head, n_head_kv, head_dim, n):
+    """As test_chunk_attention_matches_short_steps (and its bound), and every position's cache rows."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=n_head * head_dim, n_ff=256, n_head=n_head, n_head_kv=n_head_kv, n_vocab=256,
+                         n_ctx=4096)
+    engine = jf.NativeEngine(jf.Model.synthesize(cfg, type_linear=jf.F32, type_embd=jf.F32, type_output=jf.F32, seed=n_head))
+    try:
+        tokens = [int(t) for t in np.random.default_rng(n).integers(0, cfg.n_vocab, n)]
+        s, ref = engine.create_session(n), engine.create_session(n)
+        logits = s.prefill_greedy(tokens, logits=True)[1]
+        ref.prefill_greedy(tokens[:16])
+        for at in range(16, n, 16):
+            rows = engine.step_batch([ref], [tokens[at:at + 16]], logits=True)[2][0]
+        assert np.abs(logits - rows[-1]).max() <= 1e-4 * np.abs(rows[-1]).max()
+        # the second layer's keys and values follow from every row's attention: f16, so one unit in the last place more
+        for got, want in zip(s.read_kv(1, n), ref.read_kv(1, n)):
+            got, want = (np.asarray(a).view(np.float16).astype(np.float32) for a in (got, want))
+            assert np.abs(got - want).max() <= (1e-4 + 2.0 ** -10) * np.abs(want).max()
+    finally:
+        engine.close()
+
+
+@pytest.mark.parametrize("n_head,n_head_kv,head_dim,n", [(40, 8, 128, 230), (64, 8, 64, 128)])
+def test_captured_chunk_attention_replays(n_head, n_head_kv, head_dim, n):
+    """Prompts of one captured step that run without key splits: captured, then replayed with other work between, each
+    equal to the first bit for bit and to 16-row steps (bound as above)."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=n_head * head_dim, n_ff=256, n_head=n_head, n_head_kv=n_head_kv, n_vocab=256,
+                         n_ctx=4096)
+    engine = jf.NativeEngine(jf.Model.synthesize(cfg, type_linear=jf.F32, type_embd=jf.F32, type_output=jf.F32, seed=3))
+    try:
+        tokens = [int(t) for t in np.random.default_rng(n).integers(0, cfg.n_vocab, n)]
+        ref = engine.create_session(n)
+        ref.prefill_greedy(tokens[:16])
+        for at in range(16, n, 16):
+            rows = engine.step_batch([ref], [tokens[at:at + 16]], logits=True)[2][0]
+        runs = []
+        for _ in range(4):
+            s = engine.create_session(n + 4)
+            runs.append(s.prefill_greedy(tokens, logits=True)[1])
+            s.decode_greedy(1)
+            engine.matmul("blk.0.ffn_up.weight", np.ones((1, cfg.n_embd), np.float32), cfg.n_ff)
+            s.close()
+        assert np.abs(runs[0] - rows[-1]).max() <= 1e-4 * np.abs(rows[-1]).max()
+        assert all(np.array_equal(runs[0].view(np.uint32), r.view(np.uint32)) for r in runs)
+    finally:
+        engine.close()
+
+
+# 4096 q|k|v rows x 3072 at 700 rows take the 128-token tiles, their down projection the 64-token ones, 300 rows and the
+# 1280-wide model the 32-token ones.
+@pytest.mark.parametrize("n_head,n_head_kv,head_dim,n_ff", [(24, 4, 128, 2048), (20, 4, 64, 1536)], ids=["128", "64"])
+@pytest.mark.parametrize("t", TYPES, ids=[jf.TYPE_NAMES[t] for t in TYPES])
+def test_long_step_epilogues_equal_short_steps(t, n_head, n_head_kv, head_dim, n_ff):
+    """Rotated queries and keys, biases, transposed values, SwiGLU and residual adds of long steps: the caches of both
+    layers equal those of the same tokens in 8-row steps bit for bit. The first layer's attention output matrix is zero,
+    so that the second layer's rows do not depend on the attention's order of keys."""
+    cfg = jf.ModelConfig(n_layer=2, n_embd=n_head * head_dim, n_ff=n_ff, n_head=n_head, n_head_kv=n_head_kv, n_vocab=256,
+                         n_ctx=1024)
+    source = jf.Model.synthesize(cfg, type_linear=t, type_embd=jf.Q8_0, type_output=jf.Q8_0, seed=11)
+
+    def tensors():
+        for name in source.tensor_names():
+            info, data = source.tensor(name), source.tensor_bytes(name)
+            if name.endswith(".bias"):
+                data = np.random.default_rng(len(data)).standard_normal(len(data) // 4).astype(np.float32).tobytes()
+            yield name, info["type"], info["shape"], bytes(len(data)) if name == "blk.0.attn_output.weight" else data
+
+    engine = jf.NativeEngine(jf.Model.build(cfg, tensors()))
+    try:
+        for n in (300, 700):
+            tokens = [int(v) for v in np.random.default_rng(n).integers(0, cfg.n_vocab, n)]
+            s, ref = engine.create_session(n), engine.create_session(n)
+            s.prefill_greedy(tokens)
+            ref.prefill_greedy(tokens[:8])
+            for at in range(8, n, 8):
+                engine.step_batch([ref], [tokens[at:at + 8]])
+            for layer in (0, 1):
+                for what, got, want in zip("kv", s.read_kv(layer, n), ref.read_kv(layer, n)):
+                    assert np.array_equal(np.asarray(got), np.asarray(want)), f"{n} rows, layer {layer}: {what}"
+            s.close()
+            ref.close()
+    finally:
+        engine.close()

@@ -51,7 +51,7 @@ def test_stage_engines_hold_their_layer_ranges(staged):
 
 @pytest.mark.parametrize("n_prompt", [5, 300])
 def test_three_stage_pipeline_equals_full_model(staged, n_prompt):
-    """Prefill in chunks (300 rows > the 256-row chunk) and six decode steps
+    """Prefill (5 rows, a captured step; 300, beyond one step) and six decode steps
     through three stages give the full model's greedy ids; the middle
     stage's output equals what the last stage reads, row for row."""
     full, stages = staged
@@ -72,6 +72,42 @@ def test_three_stage_pipeline_equals_full_model(staged, n_prompt):
         assert got == want, f"decode step {step}"
         tok = want
     assert [si.position() for si in s] == [ref.position()] * 3
+
+
+def test_stage_prefill_of_several_chunks():
+    """A 2200-row prompt (chunks of 1152 and 1048 rows) through three stages gives the full model's greedy id and
+    continuation; every stage's rows equal those of the prompt's first 1500 rows run alone (one chunk) and of the prompt
+    cut into 384-row chunks beside a stepping session, bit for bit."""
+    cfg = jf.ModelConfig(n_layer=4, n_embd=512, n_ff=1536, n_head=8, n_head_kv=2, n_vocab=8192, n_ctx=4096)
+    model = jf.Model.synthesize(cfg, type_linear=jf.Q4_K, type_embd=jf.Q4_K, type_output=jf.Q6_K, seed=6)
+    full, stages = jf.NativeEngine(model), [jf.NativeEngine(model.slice(a, b)) for a, b in RANGES]
+    try:
+        prompt, short = _prompt(2200), 1500
+
+        def bits(a):
+            return a.view(np.uint32)
+
+        s = [e.create_session(2210) for e in stages]
+        a0 = s[0].prefill_stage(tokens=prompt)
+        a1 = s[1].prefill_stage(activations=a0)
+        tok = s[2].prefill_stage(activations=a1)
+        ref = full.create_session(2210)
+        assert ref.prefill_greedy(prompt) == tok
+        for step in range(4):
+            want = ref.decode_greedy(tok)
+            x = s[1].decode_stage(activation=s[0].decode_stage(token=tok))
+            assert s[2].decode_stage(activation=x) == want, f"decode step {step}"
+            tok = want
+        assert np.array_equal(bits(stages[0].create_session(short).prefill_stage(tokens=prompt[:short])), bits(a0[:short]))
+        assert np.array_equal(bits(stages[1].create_session(short).prefill_stage(activations=a0[:short])), bits(a1[:short]))
+        # s[0] and s[1] step just before: the chunks are cut
+        s[0].decode_stage(token=tok)
+        assert np.array_equal(bits(stages[0].create_session(2200).prefill_stage(tokens=prompt)), bits(a0))
+        s[1].decode_stage(activation=a0[:1])
+        assert np.array_equal(bits(stages[1].create_session(2200).prefill_stage(activations=a0)), bits(a1))
+    finally:
+        for e in stages + [full]:
+            e.close()
 
 
 def test_stage_activations_match_the_oracle(staged):
