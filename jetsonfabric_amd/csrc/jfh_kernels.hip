@@ -4183,10 +4183,10 @@ MmRoute fold_route(uint32_t type, int n_rg, int n_tt) {
     // one row group per work-group only while that is at most a work-group per CU
     if (n_rg * n_tt <= kCus) return {MmKernel::kFold, 1, 1};
     // Two row groups x one or two token tiles per work-group. The time goes with the work-groups that the busiest CU
-    // runs, and a work-group of two token tiles takes 1.8 times one of one tile (median over 23 matrices, 33..256
-    // rows: Q4_K 1.80, Q2_K 1.70), for Q6_K, whose fold is the longest, 1.4 times (1.45). Q4_K: 5120 x 13824, 18 rows,
-    // 2 work-groups of one tile per CU 27 us, 1 of two 21; 3584 x 18944, 100 rows, 4 and 2: 60 and 54; 7168 x 5120,
-    // 33 rows, 3 and 2: 15.7 and 21.1.
+    // runs, and a work-group of two token tiles takes 1.8 times one of one tile (median over 16 matrices of 2560
+    // columns and more, 17..256 rows: Q4_K 1.80, Q2_K 1.70), for Q6_K, whose fold is the longest, 1.4 times (1.45).
+    // Q4_K: 5120 x 13824, 18 rows, 2 work-groups of one tile per CU 27 us, 1 of two 21; 3584 x 18944, 100 rows, 4 and
+    // 2: 60 and 54; 7168 x 5120, 33 rows, 3 and 2: 15.7 and 21.1.
     const int pairs = (n_rg + 1) / 2;
     const int one = (pairs * n_tt + kCus - 1) / kCus, two = (pairs * ((n_tt + 1) / 2) + kCus - 1) / kCus;
     const int tenths = type == 13 ? 14 : 18;
@@ -4207,8 +4207,8 @@ MmRoute mm_route(uint32_t type, uint32_t rows, uint32_t cols, int32_t n_tok) {
         while (tiles > 1 && n_rg * ((n_tt + tiles - 1) / tiles) < kWideMinWgs) --tiles;
         // Q8_0 is bound by its float step per 32-value block. On grids too small for two token tiles the one-tile
         // long-step form takes about 1.15 us of latency per K tile and 0.15 us more per work-group of the busiest CU,
-        // the K-split form 0.3 us per K tile and work-group and 5 us for its cross-wave sums (fitted to 21 matrices,
-        // 33..2048 rows). 1536 x 8960, 333 rows: 47 us against 55, 256 rows 47 and 37; 4608 x 3584, 100 rows: 20.4 and
+        // the K-split form 0.3 us per K tile and work-group and 5 us for its cross-wave sums (fitted to 20 matrices,
+        // 17..2048 rows). 1536 x 8960, 333 rows: 47 us against 55, 256 rows 47 and 37; 4608 x 3584, 100 rows: 20.4 and
         // 27.9; 5120 x 27648, 100 rows: 181 and 167.
         auto per_cu = [](int n) { return (n + kCus - 1) / kCus; };
         const int nb = static_cast<int>(cols) / 256, split_wgs = n_rg * ((n_tt + tiles - 1) / tiles);

@@ -172,7 +172,7 @@ struct GemvArgs {
 void set_launch_events(hipEvent_t start, hipEvent_t stop);
 void launch_embed(const DMat& table, const StepDev* step, float* h, int32_t n_rows, int32_t H,
                   unsigned long long* best, int32_t n_best, hipStream_t stream);
-// Matmul of up to kMaxRows token rows (in groups of 8) against one matrix.
+// Matmul of any number of token rows against one matrix (in groups of 8, of kQuadGroupRows in token quads).
 void launch_gemv(const GemvArgs& a, hipStream_t stream);
 // Quantizes n_rows float rows of K values (K % 256 == 0) into `out` (blocks of out.blk).
 void launch_quantize(const float* x, int32_t stride, int32_t n_rows, const Act8& out, hipStream_t stream);
