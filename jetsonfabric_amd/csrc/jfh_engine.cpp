@@ -77,13 +77,15 @@ CachePool::~CachePool() {
 }
 
 hipError_t CachePool::allocate(void** p, size_t bytes) {
-    if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
-    (void) hipGetLastError();
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
     {
         std::lock_guard lock(pools().mutex);
         for (CachePool* pool : pools().list) pool->drain();
     }
-    return hipMalloc(p, bytes);
+    e = hipMalloc(p, bytes);
+    (void) hipGetLastError();  // the caller gets the error: the next launch is not to report it
+    return e;
 }
 
 CachePool::Buffer CachePool::take(size_t bytes) {

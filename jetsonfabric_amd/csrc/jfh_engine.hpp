@@ -37,9 +37,9 @@ class Session;
 // (qwen2_architecture.cpp:800-823, 1040-1054).
 // Host-side breakdown of a prefill (PrefillMetrics, native_inference.hpp:71-78):
 // graph capture and instantiation of step shapes met for the first time
-// (planning; none for the chunks of a prompt longer than a step), building and uploading the step descriptors (host input), the
-// device time of the step graphs (compute, HIP events around each launch) and
-// of the result copies (output read).
+// (planning; none for the chunks of a prompt longer than a step), building and
+// uploading the step descriptors (host input), the device time of the steps
+// (compute, HIP events around each) and of the result copies (output read).
 struct PrefillMetrics {
     bool plan_reused = true;         // no step graph had to be captured (chunks beyond a step run without one)
     bool attention_matrix_cores = false;  // attention on MFMA (head dim 64 or 128)

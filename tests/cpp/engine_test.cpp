@@ -96,7 +96,12 @@ void test_failed_capacity() {
         fake::memory = fake::live_bytes + limit;
         expect(refused([&] { (void) e->create_session(kCtx); }), "a session larger than the device's memory");
         fake::memory = fake::fail_from = ~size_t{0};
-        e->forward({st}, nullptr, nullptr, nullptr);
+        try {
+            e->forward({st}, nullptr, nullptr, nullptr);
+        } catch (const std::exception& err) {
+            expect(false, std::string("step after a refused session: ") + err.what());
+            continue;
+        }
         expect(s->position() == 202, "step after a refused session");
         const auto t = e->create_session(kCtx);
         e->forward({st}, nullptr, nullptr, nullptr);

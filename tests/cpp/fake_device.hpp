@@ -15,7 +15,9 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <stdexcept>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace fake {
@@ -28,6 +30,7 @@ inline size_t memory = ~size_t{0};        // ... and those that would exceed thi
 inline double clock_ms = 0.0;
 inline int faults = 0;                    // copies, fills and frees outside an allocation
 inline int captures = 0;
+inline hipError_t last_error = hipSuccess;  // of a refused allocation, until it is read: a launch reports it
 inline std::atomic<uint32_t> step_rows{0};      // rows of the step being launched
 inline std::atomic<uint32_t> longest_step{0};
 inline std::atomic<int> us_per_256_rows{0};     // real time a step's synchronization takes
@@ -51,6 +54,10 @@ using Work = std::vector<std::function<void()>>;
 inline Work captured;
 
 inline void launch(std::function<void()> work) {
+    if (last_error != hipSuccess) {
+        last_error = hipSuccess;
+        throw std::runtime_error("a launch reports the error of an earlier call");
+    }
     if (capturing) captured.push_back(std::move(work));
     else work();
 }
@@ -78,12 +85,15 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_t* p, int) {
     return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "fake device error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    std::lock_guard l(fake::lock);
+    return std::exchange(fake::last_error, hipSuccess);
+}
 
 hipError_t hipMalloc(void** p, size_t n) {
     std::lock_guard l(fake::lock);
     *p = nullptr;
-    if (n >= fake::fail_from || fake::live_bytes + n > fake::memory) return hipErrorOutOfMemory;
+    if (n >= fake::fail_from || fake::live_bytes + n > fake::memory) return fake::last_error = hipErrorOutOfMemory;
     *p = std::aligned_alloc(256, (n + 255) / 256 * 256);
     std::memset(*p, 0xA5, n);
     fake::live[reinterpret_cast<uintptr_t>(*p)] = n;
