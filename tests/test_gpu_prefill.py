@@ -1,6 +1,5 @@
 """Long steps: the prefill matmul tiles and the attention of whole prefill chunks."""
 import threading
-import time
 
 import numpy as np
 import pytest
@@ -137,12 +136,16 @@ def test_prompt_cut_for_other_sessions_is_the_same(n_head, n_head_kv, head_dim, 
         assert all(np.array_equal(a, b) for a, b in zip(alone, prefill()))  # it has just stepped
         s.close()
 
-        s, done, got = engine.create_session(4000), threading.Event(), []
-        decoder = threading.Thread(target=lambda: got.extend(greedy(s, 3900, done.is_set)))
+        s, started, done, got = engine.create_session(4000), threading.Event(), threading.Event(), []
+
+        def stop():  # asked before every step
+            started.set()
+            return done.is_set()
+
+        decoder = threading.Thread(target=lambda: got.extend(greedy(s, 3900, stop)))
         decoder.start()
         try:
-            while s.position() < 32:
-                time.sleep(1e-4)
+            assert started.wait(60)
             for _ in range(3):
                 assert all(np.array_equal(a, b) for a, b in zip(alone, prefill()))
         finally:
