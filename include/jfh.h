@@ -433,7 +433,7 @@ typedef struct jfh_generation_stats {
     uint32_t prefill_plan_reused;         /* no step graph had to be captured (chunks beyond a step run without one) */
     uint32_t prefill_attention_matrix_cores; /* attention on MFMA (head dim 64 or 128) */
     double prefill_planning_ms;           /* capturing and instantiating new step graphs */
-    double prefill_allocation_ms;         /* the session's KV cache allocation and clearing */
+    double prefill_allocation_ms;         /* the session's KV cache allocation and clearing (of caches from 32 MB) */
     double prefill_host_input_ms;         /* building and uploading the step descriptors */
     double prefill_compute_ms;            /* device time of the step graphs */
     double prefill_output_read_ms;        /* device time of the result copies */

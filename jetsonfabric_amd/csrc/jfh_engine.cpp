@@ -183,9 +183,10 @@ Session::Session(Engine* engine, uint32_t capacity)
     k_ = static_cast<uint16_t*>(buffer_.p);
     v_ = k_ + elems;
     // every use of the cache is ordered behind this on the engine's stream
-    hipError_t e = hipEventRecord(buffer_.clear_begin, engine->stream());
+    const bool timed = kv_bytes_ >= kTimedClearBytes;
+    hipError_t e = timed ? hipEventRecord(buffer_.clear_begin, engine->stream()) : hipSuccess;
     if (e == hipSuccess) e = hipMemsetAsync(k_, 0, kv_bytes_, engine->stream());
-    if (e == hipSuccess) e = hipEventRecord(buffer_.clear_end, engine->stream());
+    if (e == hipSuccess && timed) e = hipEventRecord(buffer_.clear_end, engine->stream());
     if (e != hipSuccess) {
         pool_->put(buffer_);
         hip_check(e, "clear KV cache");
@@ -200,6 +201,7 @@ Session::~Session() {
 
 double Session::clear_ms() const {
     float ms = 0.0F;
+    if (kv_bytes_ < kTimedClearBytes) return ms;
     hip_check(hipEventElapsedTime(&ms, buffer_.clear_begin, buffer_.clear_end), "cache clearing time");
     return ms;
 }

@@ -44,7 +44,7 @@ struct PrefillMetrics {
     bool plan_reused = true;         // no step graph had to be captured (chunks beyond a step run without one)
     bool attention_matrix_cores = false;  // attention on MFMA (head dim 64 or 128)
     double planning_ms = 0.0;
-    double allocation_ms = 0.0;      // the session's KV cache allocation and clearing
+    double allocation_ms = 0.0;      // the session's KV cache allocation and clearing (of caches from 32 MB)
     double host_input_ms = 0.0;
     double compute_ms = 0.0;
     double output_read_ms = 0.0;
@@ -116,7 +116,10 @@ public:
 private:
     friend class Engine;
     Session(Engine* engine, uint32_t capacity);
-    // Device time of the cache's clearing (once a step of the session has finished).
+    // Device time of the cache's clearing (once a step of the session has finished). Timing it takes about 12 us (7B,
+    // 4 layers, 100-row prompts 936 -> 948 us; with the events attached to a clearing kernel's dispatch 975), longer
+    // than clearing a cache of less than kTimedClearBytes, which counts as no time.
+    static constexpr uint64_t kTimedClearBytes = uint64_t{32} << 20;
     double clear_ms() const;
 
     Engine* engine_;

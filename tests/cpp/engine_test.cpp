@@ -20,9 +20,9 @@ void expect(bool ok, const std::string& what) {
 
 constexpr uint32_t kVocab = 512, kCtx = 8192, kLayers = 3, kEmbd = 512, kFf = 768, kHeads = 8, kKvHeads = 2, kDim = 64;
 
-std::unique_ptr<Engine> engine(uint32_t layer_start = 0, uint32_t layer_end = kLayers) {
+std::unique_ptr<Engine> engine(uint32_t layer_start = 0, uint32_t layer_end = kLayers, uint32_t kv_heads = kKvHeads) {
     SynthSpec spec;
-    spec.params = {kLayers, kEmbd, kFf, kHeads, kKvHeads, kCtx, kVocab, kDim, 1.0e6F, 1.0e-6F};
+    spec.params = {kLayers, kEmbd, kFf, kHeads, kv_heads, kCtx, kVocab, kDim, 1.0e6F, 1.0e-6F};
     const auto model = HostModel::synthesize(spec);
     if (layer_start == 0 && layer_end == kLayers) return std::make_unique<Engine>(*model, EngineOptions{});
     return std::make_unique<Engine>(*model->slice(layer_start, layer_end), EngineOptions{});
@@ -56,12 +56,12 @@ void test_prefill_scratch() {
     }
 }
 
-// A prefill's allocation time holds the clearing of its session's cache, in a new buffer and in one kept from a closed
-// session; its compute time does not.
+// A prefill's allocation time holds the clearing of its session's cache (48 MB), in a new buffer and in one kept from a
+// closed session; its compute time does not.
 void test_allocation_time() {
-    const auto e = engine();
+    const auto e = engine(0, kLayers, kHeads);
     for (int i = 0; i < 3; ++i) {
-        const auto s = e->create_session(3000);
+        const auto s = e->create_session(kCtx);
         const double clearing = 100.0 * static_cast<double>(s->kv_bytes()) / (1 << 20);
         e->prefill(*s, prompt(2500).data(), 2500, nullptr);
         const PrefillMetrics& m = s->prefill_metrics();
