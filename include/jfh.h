@@ -294,8 +294,8 @@ jfh_status jfh_session_rollback(jfh_session * session, uint32_t n);
  * count per session (may be NULL), logits (may be NULL) sum(lengths) *
  * n_vocab floats, the rows in the order of out_tokens. A step holds at most
  * 256 token rows (JFH_STATUS_INVALID_ARGUMENT beyond); prefills are split into
- * chunks of at most jfh_engine_info.prefill_chunk rows, shorter while another
- * session steps (the results do not depend on it), and steps on other threads
+ * chunks of at most jfh_engine_info.prefill_chunk rows, shorter while a session
+ * steps on another thread (the results do not depend on it), and those steps
  * take turns with them. */
 jfh_status jfh_engine_step_batch(jfh_engine * engine, jfh_session * const * sessions, uint32_t count,
                                  const int32_t * tokens, const uint32_t * lengths, int32_t * out_tokens,

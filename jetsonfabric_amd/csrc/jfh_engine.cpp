@@ -1024,6 +1024,7 @@ void Engine::forward(const std::vector<SeqStep>& steps, int32_t* out_tokens, int
     Turn turn(*this, Turn::kStep);
     run(steps, out_tokens, accepted, logits, act_out, nullptr, row_limit, 0);
     activity_->session = steps.back().session;
+    activity_->thread = std::this_thread::get_id();
     activity_->at_ns = std::chrono::steady_clock::now().time_since_epoch().count();
 }
 
@@ -1232,12 +1233,13 @@ uint32_t Engine::balanced_chunk(uint32_t n) const {
 // about 100 ms; while another session steps, chunks are kBusyChunk rows long, which hold it no longer than the 256-row
 // chunks of the split-key attention did (one layer at 4096 positions, 384 rows now and 256 then: 14B Q4_K 521 and
 // 599 us, 7B Q4_K 486 and 474, 32B Q2_K 717 and 1943; models of few heads longer, 1.5B 279 and 185). Another session
-// steps if one waits now or an open one stepped within kBusyNs, several times what a decode loop spends between steps.
+// steps if one waits now or an open one stepped on another thread within kBusyNs, several times what a decode loop
+// spends between steps.
 uint32_t Engine::next_chunk(uint32_t left, bool steps_between) {
     constexpr uint32_t kBusyChunk = 384;
     constexpr int64_t kBusyNs = 20'000'000;
     const bool busy = steps_.waiting > 0 ||
-                      (steps_between && activity_->session != nullptr &&
+                      (steps_between && activity_->session != nullptr && activity_->thread.load() != std::this_thread::get_id() &&
                        std::chrono::steady_clock::now().time_since_epoch().count() - activity_->at_ns < kBusyNs);
     const uint32_t chunk = balanced_chunk(left);
     return std::min(left, busy ? std::min(chunk, kBusyChunk) : chunk);

@@ -17,6 +17,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace jfh {
@@ -92,10 +93,11 @@ private:
     bool closed_ = false;
 };
 
-// The session that stepped last and when (steady_clock ns): whether a prefill shares the engine. Kept by the engine and
-// its sessions, since one may be closed on any thread or outlive its engine.
+// The session that stepped last, on which thread and when (steady_clock ns): whether a prefill shares the engine. Kept
+// by the engine and its sessions, since one may be closed on any thread or outlive its engine.
 struct StepActivity {
     std::atomic<const Session*> session{nullptr};
+    std::atomic<std::thread::id> thread{};
     std::atomic<int64_t> at_ns{0};
 };
 

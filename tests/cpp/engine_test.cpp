@@ -139,6 +139,11 @@ bool sooner_or_later(F&& f) {
     return false;
 }
 
+template <typename F>
+void elsewhere(F&& f) {
+    std::thread(f).join();
+}
+
 // A prompt alone runs in few long chunks; while another session steps, in chunks that hold the engine for 384 rows at
 // most and let every waiting step pass.
 void test_prefill_shares_the_engine() {
@@ -164,14 +169,16 @@ void test_prefill_shares_the_engine() {
         e->prefill(*other, ids.data(), 300, nullptr);
         expect(chunks() == 3, "chunks beside a session that does not step");
         step(*other);
+        expect(chunks() == 3, "chunks after a step of the same thread");
+        elsewhere([&] { step(*other); });
         expect(chunks(false) == 3, "chunks of a caller that lets no session step meanwhile");
         expect(sooner_or_later([&] {
-                   step(*other);
+                   elsewhere([&] { step(*other); });
                    return chunks() > 3;
                }), "chunks beside a session that has just stepped");
         std::this_thread::sleep_for(std::chrono::milliseconds(40));
         expect(chunks() == 3, "chunks beside a session that stepped long ago");
-        step(*other);
+        elsewhere([&] { step(*other); });
     }
     expect(chunks() == 3, "chunks after the other session was closed");
 
@@ -214,7 +221,7 @@ void test_stage_rows() {
             uint32_t chunks = 0;
             const uint32_t want = busy ? (n + 383) / 384 : (n + 2047) / 2048;
             const bool cut = sooner_or_later([&] {
-                if (busy) e->stage_decode(*other, nullptr, rows.data(), out.data());
+                if (busy) elsewhere([&] { e->stage_decode(*other, nullptr, rows.data(), out.data()); });
                 const auto s = e->create_session(n);
                 std::fill(out.begin(), out.end(), -1.0F);
                 e->stage_prefill(*s, nullptr, rows.data(), n, out.data());

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -100,10 +101,16 @@ def test_stage_prefill_of_several_chunks():
             tok = want
         assert np.array_equal(bits(stages[0].create_session(short).prefill_stage(tokens=prompt[:short])), bits(a0[:short]))
         assert np.array_equal(bits(stages[1].create_session(short).prefill_stage(activations=a0[:short])), bits(a1[:short]))
-        # s[0] and s[1] step just before: the chunks are cut
-        s[0].decode_stage(token=tok)
+        # s[0] and s[1] step just before on another thread: the chunks are cut
+
+        def elsewhere(step):
+            thread = threading.Thread(target=step)
+            thread.start()
+            thread.join()
+
+        elsewhere(lambda: s[0].decode_stage(token=tok))
         assert np.array_equal(bits(stages[0].create_session(2200).prefill_stage(tokens=prompt)), bits(a0))
-        s[1].decode_stage(activation=a0[:1])
+        elsewhere(lambda: s[1].decode_stage(activation=a0[:1]))
         assert np.array_equal(bits(stages[1].create_session(2200).prefill_stage(activations=a0)), bits(a1))
     finally:
         for e in stages + [full]:
